@@ -7,18 +7,18 @@
 // n1 = min(m, n) / 2, factor the left block, apply its row interchanges to
 // the right block, solve A12 = L11^-1 A12 (unit lower), update
 // A22 -= A21 A12, factor A22 and apply its interchanges to the left block.
-// Blocks of up to 8 columns are one kernel (the same eliminations with
-// rank-1 updates in place of the GEMMs of that width), which keeps the
-// launch count near 5 per 8 columns instead of 5 per column.  Such a leaf
-// is held in registers: by one work-group up to 4096 rows, by one
-// work-group per 2048 rows with a grid barrier per column above that.  Pivots are
-// kept as global rows throughout (the reference shifts them by n1 after
-// each recursive call).  Everything is enqueued on the caller's stream;
-// pivots and info stay on the device.
+// Panels of up to 64 columns are one kernel (the same eliminations with
+// rank-1 updates in place of the GEMMs of that width), held in registers by
+// up to 128 work-groups that exchange one pivot row per column (32 columns
+// above 32,768 rows, 16 above 65,536; past 131,072 rows 8 columns in global
+// memory).  Pivots are kept as global rows throughout (the reference shifts
+// them by n1 after each recursive call).  Everything is enqueued on the
+// caller's stream; pivots and info stay on the device.
 #include <hip/hip_runtime.h>
 
 #include <limits>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/nla.h"
@@ -41,8 +41,10 @@ constexpr int PIV_THREADS = 1024;
 // the recursion's GEMM updates do at this width).  m == 1 is the reference's
 // row case (src/lu.jl:216-221).  Pivots are written 1-based with the leaf's
 // row offset r0 added (its rows start on the diagonal, r0 = its first
-// column); info takes the first zero pivot's global column.
-constexpr int LEAF_COLS = 8;
+// column); info takes the first zero pivot's global column.  Used for blocks
+// that the register panels do not take (up to LEAF_COLS columns) and to redo
+// a panel (up to LEAF_COLS_MAX) whose groups did not meet.
+constexpr int LEAF_COLS = 8, LEAF_COLS_MAX = 64;
 constexpr int LEAF_WAVES = PIV_THREADS / 64;
 
 // (|a|, signed a, row) of the larger |a|, ties to the smaller row.
@@ -70,7 +72,7 @@ __device__ __forceinline__ void lu_leaf_body(int64_t m, int n, T *__restrict__ A
                              int64_t *__restrict__ info, int64_t r0) {
     __shared__ T s_val[2][LEAF_WAVES], s_sgn[2][LEAF_WAVES];
     __shared__ int64_t s_row[2][LEAF_WAVES];
-    __shared__ T s_u[LEAF_COLS];  // row j of the leaf after the interchange
+    __shared__ T s_u[LEAF_COLS_MAX];  // row j of the leaf after the interchange
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int kmax = (int)(m < n ? m : n);
     // partial maxima of column 0 (each later column's are taken in the
@@ -124,9 +126,9 @@ __device__ __forceinline__ void lu_leaf_body(int64_t m, int n, T *__restrict__ A
         if (a != T(0)) {
             // scale column j below the pivot, update the columns to its right
             // and take the partial maxima of column j + 1.  Rows go in chunks
-            // of RU per thread; every load of a chunk (column j and all the
-            // columns to its right) is issued before its first store, with
-            // addresses clamped to row / column j and results masked.
+            // of RU per thread and columns in chunks of NC; every load of a
+            // chunk is issued before its first store, with addresses clamped
+            // to row / column j and results masked.
             constexpr int RU = 4, NC = LEAF_COLS - 1;
             const bool recip = fabs(a) >= std::numeric_limits<T>::min();
             const T r = T(1) / a;
@@ -138,34 +140,35 @@ __device__ __forceinline__ void lu_leaf_body(int64_t m, int n, T *__restrict__ A
                     l[u] = cj[i < m ? i : j];
                 }
 #pragma unroll
-                for (int q = 0; q < NC; ++q) {
-                    const int c = j + 1 + q;
-                    const T *cc = A + (int64_t)(c < n ? c : j) * lda;
-#pragma unroll
-                    for (int u = 0; u < RU; ++u) {
-                        const int64_t i = i0 + (int64_t)u * PIV_THREADS;
-                        x[q][u] = cc[i < m ? i : j];
-                    }
-                }
-#pragma unroll
                 for (int u = 0; u < RU; ++u) {
                     const int64_t i = i0 + (int64_t)u * PIV_THREADS;
                     l[u] = recip ? l[u] * r : l[u] / a;
                     if (i < m) cj[i] = l[u];
                 }
+                for (int c0 = j + 1; c0 < n; c0 += NC) {
 #pragma unroll
-                for (int q = 0; q < NC; ++q) {
-                    const int c = j + 1 + q;
-                    if (c >= n) break;
-                    T *cc = A + (int64_t)c * lda;
-                    const T uc = s_u[c];
+                    for (int q = 0; q < NC; ++q) {
+                        const T *cc = A + (int64_t)(c0 + q < n ? c0 + q : j) * lda;
 #pragma unroll
-                    for (int u = 0; u < RU; ++u) {
-                        const int64_t i = i0 + (int64_t)u * PIV_THREADS;
-                        if (i < m) {
-                            const T y = x[q][u] - l[u] * uc;
-                            cc[i] = y;
-                            if (q == 0) better(bv, bs, bi, (T)fabs(y), y, i);
+                        for (int u = 0; u < RU; ++u) {
+                            const int64_t i = i0 + (int64_t)u * PIV_THREADS;
+                            x[q][u] = cc[i < m ? i : j];
+                        }
+                    }
+#pragma unroll
+                    for (int q = 0; q < NC; ++q) {
+                        const int c = c0 + q;
+                        if (c >= n) break;
+                        T *cc = A + (int64_t)c * lda;
+                        const T uc = s_u[c];
+#pragma unroll
+                        for (int u = 0; u < RU; ++u) {
+                            const int64_t i = i0 + (int64_t)u * PIV_THREADS;
+                            if (i < m) {
+                                const T y = x[q][u] - l[u] * uc;
+                                cc[i] = y;
+                                if (c == j + 1) better(bv, bs, bi, (T)fabs(y), y, i);
+                            }
                         }
                     }
                 }
@@ -190,270 +193,481 @@ __global__ __launch_bounds__(PIV_THREADS) void lu_leaf_kernel(int64_t m, int n, 
     lu_leaf_body<T>(m, n, A, lda, ipiv, info, r0);
 }
 
-// The same leaf for tall blocks, spread over G work-groups of SPLIT_ROWS
-// rows each, the block held in registers from the first load to the final
-// store.  Per column: each work-group finds its candidate (first index of
-// the largest |a| among its rows at or below the diagonal) and publishes it
-// with its row, the group holding row j publishes that row, and after one
-// grid barrier every work-group takes the same winner, makes the same
-// interchange in its registers and eliminates its own rows.  The published
-// values alternate between two buffers by column parity, so a work-group
-// one column ahead never overwrites what a slower one still reads.  At most
-// 64 groups of one CU each are launched, which an idle part of the chip
+// The same factorization of a panel of up to NB columns, held in registers
+// by G work-groups of NT threads with R rows per thread from the first load
+// to the final store.  What bounds it is the chain of columns, not the
+// arithmetic, so a column is two trips through memory (the candidates, the
+// winner's row) and two work-group barriers, with everything that the next
+// candidate does not need moved off that chain:
+//   1. after the pivot row arrives, a thread first forms its entry of the
+//      next column; each wave reduces its candidate (the largest |a| among
+//      its live rows, ties to the smaller position) on DPP moves and wave 0
+//      publishes the group's;
+//   2. only then are the other columns updated, and the wave that holds the
+//      group's candidate publishes that row and the reciprocal of its pivot,
+//      while the candidates travel;
+//   3. wave 0 reads all candidates and then the winner's row.  A 64-bit word
+//      carries 32 bits of payload under a 32-bit tag that names the launch
+//      and the column, so a reader polls the data itself: no counter, no
+//      fence.  The slots alternate with the column's parity: a group
+//      publishes column j + 2 only after all groups have published j + 1,
+//      which each does after its last read of column j.
+// The register columns move down by one with the update itself
+// (a[c] = a[c + 1] - l u[c + 1]), so the column loop stays rolled and the
+// kernel small; the finished column of L goes to LDS.  Rows are not moved: a
+// row keeps its thread and carries its position, and is stored to its final
+// position at the end.
+//
+// Measured on MI355X, FP64: 166 us per 64 columns at 1,000 to 8,192 rows
+// (2.6 us per column: about 2 us in the two trips, whatever the number of
+// groups), 73 us in one group up to 128 rows; 8-column leaves with a counter
+// per column took 480 us above 4,096 rows and 256 us below, plus the
+// launches between them.  Groups of 64, 128 and 256 rows measure alike; all
+// groups on one XCD, with agent- or L2-scope words, is no faster.
+//
+// At most LU_MAX_WG groups are launched, which an idle part of the chip
 // holds at once; a cooperative launch would guarantee it, but costs about
 // 150 us once other streams have been used.  Each wait is bounded, so a
 // group that is not resident (another persistent grid holds the CUs) cannot
-// hang the others.  Every group saves its rows before the first barrier (and
-// group 0 the prior info), and a wait that runs out raises a flag; the
-// one-work-group recovery launch that follows every split leaf returns at
+// hang the others.  Every group saves its rows before its first exchange
+// (and group 0 the prior info), and a wait that runs out raises a flag; the
+// one-work-group recovery launch that follows every such panel returns at
 // once unless the flag is up, and otherwise restores the saved block and
 // factors it with the global-memory leaf, so the factorization stays exact.
-// The last group to finish resets the counters for the next launch on the
-// stream.
-// With ONE (a single work-group) the group's own winner is the pivot and
-// nothing is published: the whole leaf stays in registers with two
-// work-group barriers per column and no memory round trip.
-constexpr int SPLIT_THREADS = 256, SPLIT_RPT = 8, SPLIT_ROWS = SPLIT_THREADS * SPLIT_RPT;
-constexpr int ONE_THREADS = 512, ONE_RPT = 8, ONE_ROWS = ONE_THREADS * ONE_RPT;
-constexpr int SPLIT_MAX_WG = 64, SPLIT_SLOT = 16;  // 64-bit words per published candidate
-constexpr int SYNC_SLOTS = 64, SYNC_DIAG = SYNC_SLOTS + 2 * SPLIT_MAX_WG * SPLIT_SLOT;
-constexpr int SYNC_WORDS = SYNC_DIAG + 2 * SPLIT_SLOT;
+// A single group (ONE) exchanges nothing: one barrier per column.
+constexpr int LU_MAX_WG = 128;              // groups of one panel (two polled per lane)
+constexpr int LU_WORDS = 64;                // registers of a row: NB * R
+constexpr int SYNC_EPOCH = 0, SYNC_LEAVE = 1;
 // words 2, 3 of the buffer: the timeout flag and the info value saved before
-// the leaf; after SYNC_WORDS: the saved block, column c at c * SAVE_LD
+// the panel; then, for both parities, the groups' candidates (three arrays of
+// one word per group, so that a poll of all of them touches few lines) and
+// their rows; then the saved block (column c at c * m)
 constexpr int SYNC_FLAG = 2, SYNC_INFO = 3;
-constexpr int64_t SAVE_LD = (int64_t)SPLIT_ROWS * SPLIT_MAX_WG;
-constexpr int64_t SYNC_BYTES = SYNC_WORDS * 8 + SAVE_LD * LEAF_COLS * 8;
+constexpr int SYNC_SLOTS = 64, HEAD_WORDS = 3 * LU_MAX_WG, ROW_WORDS = 136;
+constexpr int PAR_WORDS = HEAD_WORDS + LU_MAX_WG * ROW_WORDS;
+constexpr int SYNC_WORDS = SYNC_SLOTS + 2 * PAR_WORDS;
+constexpr int64_t PANEL_M_MAX = 256 * LU_MAX_WG;  // rows of a 64-column panel
+constexpr int64_t SYNC_BYTES = SYNC_WORDS * 8 + PANEL_M_MAX * LU_WORDS * 8;
 constexpr int64_t SPLIT_SPIN_LIMIT = int64_t(1) << 20;  // about a second of polling
 
 __device__ inline void st_agent(uint64_t *p, uint64_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ inline uint64_t ld_agent(uint64_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ inline uint64_t dbits(double v) { return (uint64_t)__double_as_longlong(v); }
-__device__ inline double bitsd(uint64_t v) { return __longlong_as_double((long long)v); }
+__device__ inline uint64_t ld_agent(const uint64_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
-template <typename T, int NT, int RPT, bool ONE>
-__global__ __launch_bounds__(NT) void lu_leaf_reg_kernel(int64_t m, int n, T *__restrict__ A, int64_t lda,
-                                                         int64_t *__restrict__ ipiv, int64_t *__restrict__ info,
-                                                         int64_t r0, uint64_t *__restrict__ sync,
-                                                         int64_t spin_limit) {
-    constexpr int W = NT / 64, ROWS = NT * RPT;
-    __shared__ T s_val[W], s_sgn[W];
-    __shared__ int64_t s_row[W];
-    __shared__ T s_u[LEAF_COLS], s_o[LEAF_COLS];  // candidate / pivot row, row j before the interchange
-    __shared__ T s_a;
-    __shared__ int64_t s_p;
-    __shared__ int s_fail;
+// Columns of the register panel for m rows (a row's NB * R registers are the
+// same for every height), 0 where the panel does not take them.
+inline int panel_cols(int64_t m) {
+    return m <= PANEL_M_MAX ? 64 : (m <= 2 * PANEL_M_MAX ? 32 : (m <= 4 * PANEL_M_MAX ? 16 : 0));
+}
+
+__device__ __forceinline__ double lane_double(double v, int l) {
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, l);
+    const unsigned hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), l);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// The wave's largest v (no NaN; lanes without a row hold -2) and the
+// smallest position that has it; returns its lane.  Six DPP steps instead
+// of shuffles through LDS; several lanes with the same value are rare (a
+// zero column), so their positions are compared one by one.
+__device__ __forceinline__ int wave_best(double v, int pos, double &best, int &bpos) {
+    double x = v;
+#define NLA_DPP_MAX(CTRL)                                                                                   \
+    {                                                                                                       \
+        const uint64_t b = (uint64_t)__double_as_longlong(x), id = (uint64_t)__double_as_longlong(-2.0);    \
+        const unsigned lo = __builtin_amdgcn_update_dpp((int)id, (int)b, CTRL, 0xf, 0xf, false);            \
+        const unsigned hi = __builtin_amdgcn_update_dpp((int)(id >> 32), (int)(b >> 32), CTRL, 0xf, 0xf, false); \
+        x = fmax(x, __longlong_as_double((long long)(((uint64_t)hi << 32) | lo)));                          \
+    }
+    NLA_DPP_MAX(0x111)  // row_shr 1, 2, 4, 8
+    NLA_DPP_MAX(0x112)
+    NLA_DPP_MAX(0x114)
+    NLA_DPP_MAX(0x118)
+    NLA_DPP_MAX(0x142)  // row_bcast 15, 31
+    NLA_DPP_MAX(0x143)
+#undef NLA_DPP_MAX
+    best = lane_double(x, 63);
+    uint64_t who = best > -2.0 ? __ballot(v == best) : 1;  // a wave without rows: lane 0's position (none)
+    int l = __ffsll((unsigned long long)who) - 1;
+    bpos = __builtin_amdgcn_readlane(pos, l);
+    for (who &= who - 1; who; who &= who - 1) {
+        const int l2 = __ffsll((unsigned long long)who) - 1;
+        const int p2 = __builtin_amdgcn_readlane(pos, l2);
+        if (p2 < bpos) {
+            bpos = p2;
+            l = l2;
+        }
+    }
+    return l;
+}
+
+template <typename T, int NB, int R, int NT, bool ONE>
+__global__ __launch_bounds__(NT) void lu_panel_kernel(int m, int n, T *__restrict__ A, int64_t lda,
+                                                      int64_t *__restrict__ ipiv, int64_t *__restrict__ info,
+                                                      int64_t r0, uint64_t *__restrict__ sync, int64_t spin_limit) {
+    constexpr int W = NT / 64, ROWS = NT * R;
+    static_assert(NB <= 64 && NB % 16 == 0, "a wave publishes one row");
+    __shared__ T s_l[NB][ROWS];                                       // finished columns (and rows of U)
+    __shared__ __attribute__((aligned(16))) T s_row[2][W][NB + 2];    // each wave's candidate row, entry c at c + 1
+    __shared__ __attribute__((aligned(16))) T s_u[2][NB + 2];         // the pivot row, entry c at c + 1; 1 / pivot at 0
+    __shared__ double s_v[2][W];
+    __shared__ int s_pos[2][W], s_src[2][W];
+    __shared__ int s_p[2], s_own[2], s_fail;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int G = (int)gridDim.x, g = (int)blockIdx.x;
-    const int64_t first = (int64_t)g * ROWS;  // this group's rows: [first, first + ROWS)
-    const int64_t base = first + t;
-    const int kmax = (int)(m < n ? m : n);
-    uint64_t *arrive = sync, *leave = sync + 1;
-    T a[RPT][LEAF_COLS];
+    const int first = g * ROWS;
+    const int kmax = m < n ? m : n;
+    T a[R][NB];
+    int pos[R];  // the row's position; -1 - position once it is a pivot row (or past m)
 #pragma unroll
-    for (int r = 0; r < RPT; ++r) {
-        const int64_t i = base + (int64_t)r * NT;
+    for (int r = 0; r < R; ++r) {
+        const int i = first + t + r * NT;
 #pragma unroll
-        for (int c = 0; c < LEAF_COLS; ++c) a[r][c] = (i < m && c < n) ? A[i + (int64_t)c * lda] : T(0);
+        for (int c = 0; c < NB; ++c) a[r][c] = (i < m && c < n) ? A[i + (int64_t)c * lda] : T(0);
+        pos[r] = i < m ? i : -1 - i;
     }
     if (t == 0) s_fail = 0;
+    unsigned epoch = 0;
     if constexpr (!ONE) {
         // the block as it was, for the recovery launch
         T *save = reinterpret_cast<T *>(sync + SYNC_WORDS);
 #pragma unroll
-        for (int r = 0; r < RPT; ++r) {
-            const int64_t i = base + (int64_t)r * NT;
-            if (i < m) {
+        for (int r = 0; r < R; ++r) {
+            if (pos[r] >= 0) {
 #pragma unroll
-                for (int c = 0; c < LEAF_COLS; ++c)
-                    if (c < n) save[i + (int64_t)c * SAVE_LD] = a[r][c];
+                for (int c = 0; c < NB; ++c)
+                    if (c < n) save[pos[r] + (int64_t)c * m] = a[r][c];
             }
         }
-        // only group 0 writes info, and the same thread arrives first at
-        // every barrier after this store
         if (g == 0 && t == 0) st_agent(sync + SYNC_INFO, (uint64_t)*info);
+        epoch = (unsigned)ld_agent(sync + SYNC_EPOCH);
     }
-    bool failed = false;  // lane 0 of wave 0: a wait ran out; later ones are skipped
-#pragma unroll
-    for (int j = 0; j < LEAF_COLS; ++j) {
-        if (j >= kmax) break;
+    // The group's candidate of column j from the threads' entries x of it:
+    // (|pivot|, position, wave, LDS row); one barrier.  br: the candidate's
+    // row of this thread, wl: this wave's candidate lane.
+    double gv;
+    int gp, gw, gs, br, wl;
+    auto candidate = [&](int j, const T *x, auto write_row) {
         const int par = j & 1;
-        T bv = T(-1), bs = T(0);
-        int64_t bi = m;
+        double bv = -2.0;
+        int bp = 0x7fffffff;
+        br = 0;
 #pragma unroll
-        for (int r = 0; r < RPT; ++r) {
-            const int64_t i = base + (int64_t)r * NT;
-            if (i >= j && i < m) better(bv, bs, bi, (T)fabs(a[r][j]), a[r][j], i);
+        for (int r = 0; r < R; ++r) {
+            double v = fabs((double)x[r]);
+            v = v >= 0.0 ? v : -1.0;  // a NaN only wins where there is nothing else: the first live row stays
+            v = pos[r] >= 0 ? v : -2.0;
+            if (v > bv || (R > 1 && v == bv && pos[r] >= 0 && pos[r] < bp)) {
+                bv = v;
+                bp = pos[r];
+                br = r;
+            }
         }
-        wave_argmax(bv, bs, bi);
-        if (lane == 0) {
-            s_val[wv] = bv;
-            s_sgn[wv] = bs;
-            s_row[wv] = bi;
+        double wbest;
+        int wpos;
+        wl = wave_best(bv, bp, wbest, wpos);
+        if (lane == wl) {
+            s_v[par][wv] = wbest;
+            s_pos[par][wv] = wpos;
+            s_src[par][wv] = t + br * NT;
+            write_row();
         }
         __syncthreads();
-        T pv = T(-1), ps = T(0);
-        int64_t pi = m;
+        gv = s_v[par][0];
+        gp = s_pos[par][0];
+        gs = s_src[par][0];
+        gw = 0;
 #pragma unroll
-        for (int w = 0; w < W; ++w) better(pv, ps, pi, s_val[w], s_sgn[w], s_row[w]);
-#pragma unroll
-        for (int r = 0; r < RPT; ++r) {
-            const int64_t i = base + (int64_t)r * NT;
-            if (i == pi) {
-#pragma unroll
-                for (int c = 0; c < LEAF_COLS; ++c) s_u[c] = a[r][c];
+        for (int w = 1; w < W; ++w) {
+            const double v = s_v[par][w];
+            const int q = s_pos[par][w], sr = s_src[par][w];
+            if (v > gv || (v == gv && v > -2.0 && q < gp)) {
+                gv = v;
+                gp = q;
+                gs = sr;
+                gw = w;
             }
-            if (i == j) {
+        }
+    };
+    // this thread's candidate row (entry c at c + 1), by its lane
+    auto put_row = [&](T *dst, auto width) {
+        constexpr int WD = decltype(width)::value;
 #pragma unroll
-                for (int c = 0; c < LEAF_COLS; ++c) s_o[c] = a[r][c];
+        for (int c = 0; c < WD; ++c) {
+            T x = a[0][c];
+#pragma unroll
+            for (int r = 1; r < R; ++r) {
+                T y = a[r][c];
+                asm("" : "+v"(y));  // a select of values: one of addresses would put the rows in memory
+                if (br == r) x = y;
             }
+            dst[c + 1] = x;
         }
-        __syncthreads();
-        int64_t p = pi;
-        T av = ps;
-        if constexpr (!ONE) {
-            if (wv == 0) {
-                uint64_t *slot = sync + SYNC_SLOTS + (par * SPLIT_MAX_WG + g) * SPLIT_SLOT;
-                if (lane == 0) {
-                    st_agent(slot + 0, dbits((double)pv));
-                    st_agent(slot + 1, dbits((double)ps));
-                    st_agent(slot + 2, (uint64_t)pi);
-                }
-                if (lane < LEAF_COLS) {
-                    st_agent(slot + 4 + lane, dbits(pi < m ? (double)s_u[lane] : 0.0));
-                    if (j >= first && j < first + ROWS)
-                        st_agent(sync + SYNC_DIAG + par * SPLIT_SLOT + lane, dbits((double)s_o[lane]));
-                }
-                if (lane == 0) {
-                    // grid barrier: arrival count reaches G * (j + 1)
-                    __hip_atomic_fetch_add(arrive, (uint64_t)1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-                    const uint64_t target = (uint64_t)G * (uint64_t)(j + 1);
-                    int64_t spins = 0;
-                    while (!failed && ld_agent(arrive) < target) {
-                        if (++spins > spin_limit) {
-                            failed = true;
-                            s_fail = 1;
-                            break;
-                        }
-                        __builtin_amdgcn_s_sleep(1);
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                }
-                // every lane reads one group's candidate (and lanes < LEAF_COLS
-                // row j), then the wave reduces to the winner; ties go to the
-                // smaller row, as within a group
-                double cv = -1.0, cs = 0.0, crow[LEAF_COLS];
-                int64_t ci = m;
-                if (lane < G) {
-                    uint64_t *sl = sync + SYNC_SLOTS + (par * SPLIT_MAX_WG + lane) * SPLIT_SLOT;
-                    cv = bitsd(ld_agent(sl + 0));
-                    cs = bitsd(ld_agent(sl + 1));
-                    ci = (int64_t)ld_agent(sl + 2);
-#pragma unroll
-                    for (int c = 0; c < LEAF_COLS; ++c) crow[c] = bitsd(ld_agent(sl + 4 + c));
-                } else {
-#pragma unroll
-                    for (int c = 0; c < LEAF_COLS; ++c) crow[c] = 0.0;
-                }
-                const double rowj = lane < LEAF_COLS ? bitsd(ld_agent(sync + SYNC_DIAG + par * SPLIT_SLOT + lane)) : 0.0;
-                wave_argmax(cv, cs, ci);
-                // the winning candidate's lane is the group holding row ci
-                const int wl = ci < m ? (int)(ci / ROWS) : 0;
-                double u = 0.0;
-#pragma unroll
-                for (int c = 0; c < LEAF_COLS; ++c) {
-                    const double x = __shfl(crow[c], wl, 64);
-                    if (lane == c) u = x;
-                }
-                if (lane == 0) {
-                    s_p = ci;
-                    s_a = (T)cs;
-                }
-                if (lane < LEAF_COLS) {
-                    s_u[lane] = (T)u;
-                    s_o[lane] = (T)rowj;
-                }
-            }
-            __syncthreads();
-            p = s_p;
-            av = s_a;
-        }
-        T u[LEAF_COLS], o[LEAF_COLS];
-#pragma unroll
-        for (int c = 0; c < LEAF_COLS; ++c) {
-            u[c] = s_u[c];
-            o[c] = s_o[c];
-        }
-        if (p >= m) {  // no finite maximum (all NaN): keep row j
-            p = j;
-            av = o[j];
-#pragma unroll
-            for (int c = 0; c < LEAF_COLS; ++c) u[c] = o[c];
-        }
+    };
+    // Column j eliminated with pivot row u (position p, LDS row src of this
+    // group if own).  Each thread's entry of column j + 1 comes first
+    // (next()), then the other columns.
+    auto eliminate = [&](int j, int p, bool own, int src, const T *u, bool have_rc, auto width, auto next) {
+        constexpr int WD = decltype(width)::value;
+        const T av = u[1];
         if (g == 0 && t == 0) {
             ipiv[j] = r0 + p + 1;
             if (av == T(0) && *info == 0) *info = r0 + j + 1;
         }
+        T x[R];
         if (av != T(0)) {
-            const bool swap = p != j;
+            // the pivot row is row j of U from here on
+            if (own && wv == W - 1 && lane < WD && j + lane < NB) s_l[j + lane][src] = u[lane + 1];
             const bool recip = fabs(av) >= std::numeric_limits<T>::min();
-            const T rc = T(1) / av;
+            const T rc = have_rc ? u[0] : T(1) / av, u1 = u[2];
+            T l[R];
 #pragma unroll
-            for (int r = 0; r < RPT; ++r) {
-                const int64_t i = base + (int64_t)r * NT;
-                if (swap && i == j) {
+            for (int r = 0; r < R; ++r) {
+                if (pos[r] == p) pos[r] = -1 - j;
+                else if (pos[r] == j) pos[r] = p;
+                l[r] = recip ? a[r][0] * rc : a[r][0] / av;
+                x[r] = a[r][1] - l[r] * u1;
+            }
+            next(x);
 #pragma unroll
-                    for (int c = 0; c < LEAF_COLS; ++c) a[r][c] = u[c];
-                } else if (swap && i == p) {
+            for (int r = 0; r < R; ++r) {
+                if (pos[r] >= 0) s_l[j][t + r * NT] = l[r];
+                a[r][0] = x[r];
+            }
 #pragma unroll
-                    for (int c = 0; c < LEAF_COLS; ++c) a[r][c] = o[c];
+            for (int c = 1; c + 1 < WD; ++c) {
+                const T uc = u[c + 2];
+#pragma unroll
+                for (int r = 0; r < R; ++r) a[r][c] = a[r][c + 1] - l[r] * uc;
+            }
+        } else {
+            // nothing to eliminate and nothing moved: the row at position j is
+            // row j of U as it stands
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (pos[r] == j) {
+                    pos[r] = -1 - j;
+#pragma unroll
+                    for (int c = 0; c < WD; ++c)
+                        if (j + c < NB) s_l[j + c][t + r * NT] = a[r][c];
+                } else if (pos[r] >= 0) {
+                    s_l[j][t + r * NT] = a[r][0];
                 }
-                if (i > j && i < m) {
-                    const T l = recip ? a[r][j] * rc : a[r][j] / av;
-                    a[r][j] = l;
+                x[r] = a[r][1];
+            }
+            next(x);
 #pragma unroll
-                    for (int c = j + 1; c < LEAF_COLS; ++c) a[r][c] = a[r][c] - l * u[c];
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int c = 0; c + 1 < WD; ++c) a[r][c] = a[r][c + 1];
+        }
+    };
+    // One group: column j from its own candidate; WD: register columns still
+    // in use (the panel's last columns run with narrower copies of the code).
+    auto column_one = [&](int j, auto width) {
+        const int par = j & 1;
+        T x[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) x[r] = a[r][0];
+        candidate(j, x, [&] { put_row(s_row[par][wv], width); });
+        eliminate(j, gp, true, gs, s_row[par][gw], false, width, [](const T *) {});
+    };
+    uint64_t *heads = nullptr, *rows = nullptr;
+    uint64_t tg = 0;
+    auto at_column = [&](int j) {
+        tg = (uint64_t)(epoch + (unsigned)j + 1u) << 32;
+        heads = sync + SYNC_SLOTS + (int64_t)(j & 1) * PAR_WORDS;
+        rows = heads + HEAD_WORDS;
+    };
+    auto put_head = [&]() {
+        if (wv == 0 && lane < 3) {
+            const uint64_t vb = (uint64_t)__double_as_longlong(gv);
+            st_agent(heads + lane * LU_MAX_WG + g,
+                     tg | (lane == 0 ? (vb >> 32) : (lane == 1 ? (vb & 0xffffffffu) : (uint64_t)(unsigned)gp)));
+        }
+    };
+    // the candidate's wave: the row, and the reciprocal of its first entry
+    auto send_row = [&](auto width) {
+        constexpr int WD = decltype(width)::value;
+        if (wv != gw) return;
+        T *row = s_row[0][wv];
+        if (lane == wl) put_row(row, width);
+        __builtin_amdgcn_wave_barrier();
+        uint64_t *mine = rows + (int64_t)g * ROW_WORDS;
+        const T rc = T(1) / row[1];
+        const T x = row[(lane < WD ? lane : 0) + 1];
+        if constexpr (sizeof(T) == 8) {
+            const uint64_t xb = (uint64_t)__double_as_longlong((double)x), rb = (uint64_t)__double_as_longlong((double)rc);
+            if (lane < WD) {
+                st_agent(mine + 2 * lane, tg | (xb >> 32));
+                st_agent(mine + 2 * lane + 1, tg | (xb & 0xffffffffu));
+            }
+            if (lane < 2) st_agent(mine + 2 * 64 + lane, tg | (lane == 0 ? (rb >> 32) : (rb & 0xffffffffu)));
+        } else {
+            if (lane < WD) st_agent(mine + lane, tg | __float_as_uint((float)x));
+            if (lane == 0) st_agent(mine + 64, tg | __float_as_uint((float)rc));
+        }
+    };
+    auto tagged = [&](uint64_t w) { return (w >> 32) == (tg >> 32); };
+    auto column = [&](int j, auto width) -> bool {
+        constexpr int WD = decltype(width)::value;
+        const int par = j & 1;
+        if (wv == 0) {
+            // the groups' candidates: lane l reads groups l and l + 64
+            double cv = -2.0;
+            int cp = 0x7fffffff, cg = lane;
+            bool fail = false;
+            int64_t spins = 0;
+#pragma unroll
+            for (int h = 0; h < LU_MAX_WG / 64; ++h) {
+                if (h * 64 >= G) break;
+                const int q = h * 64 + lane;
+                const uint64_t *sl = heads + (q < G ? q : g);
+                uint64_t w0, w1, w2;
+                for (;;) {
+                    w0 = ld_agent(sl);
+                    w1 = ld_agent(sl + LU_MAX_WG);
+                    w2 = ld_agent(sl + 2 * LU_MAX_WG);
+                    if (__all(tagged(w0) && tagged(w1) && tagged(w2))) break;
+                    if (++spins > spin_limit) {
+                        fail = true;
+                        break;
+                    }
+                }
+                if (fail) break;
+                const double v = __longlong_as_double((long long)((w0 << 32) | (w1 & 0xffffffffu)));
+                const int x = (int)(unsigned)w2;
+                if (q < G && (v > cv || (v == cv && x < cp))) {
+                    cv = v;
+                    cp = x;
+                    cg = q;
                 }
             }
+            int win = 0, p = 0;
+            T x = T(0), rc = T(0);
+            if (!fail) {
+                double best;
+                const int l = wave_best(cv, cp, best, p);
+                win = __builtin_amdgcn_readlane(cg, l);
+                const uint64_t *row = rows + (int64_t)win * ROW_WORDS;
+                const int e = lane < WD ? lane : 0;
+                for (;;) {
+                    bool here;
+                    if constexpr (sizeof(T) == 8) {
+                        const uint64_t h = ld_agent(row + 2 * e), o = ld_agent(row + 2 * e + 1);
+                        const uint64_t rh = ld_agent(row + 128), ro = ld_agent(row + 129);
+                        here = tagged(h) && tagged(o) && tagged(rh) && tagged(ro);
+                        x = (T)__longlong_as_double((long long)((h << 32) | (o & 0xffffffffu)));
+                        rc = (T)__longlong_as_double((long long)((rh << 32) | (ro & 0xffffffffu)));
+                    } else {
+                        const uint64_t h = ld_agent(row + e), rh = ld_agent(row + 64);
+                        here = tagged(h) && tagged(rh);
+                        x = (T)__uint_as_float((unsigned)h);
+                        rc = (T)__uint_as_float((unsigned)rh);
+                    }
+                    if (__all(here)) break;
+                    if (++spins > spin_limit) {
+                        fail = true;
+                        break;
+                    }
+                }
+            }
+            if (lane < WD) s_u[par][lane + 1] = x;
+            if (lane == 0) {
+                s_u[par][0] = rc;
+                s_p[par] = p;
+                s_own[par] = win == g ? 1 : 0;
+                if (fail) s_fail = 1;
+            }
         }
+        __syncthreads();
+        if (s_fail) return false;
+        const bool more = j + 1 < kmax;
+        eliminate(j, s_p[par], s_own[par] != 0, gs, s_u[par], true, width, [&](const T *x) {
+            if (!more) return;
+            at_column(j + 1);
+            candidate(j + 1, x, [] {});
+            put_head();
+        });
+        if (more) send_row(width);
+        return true;
+    };
+    bool good = true;
+    auto run = [&](int j, auto width) {
+        if constexpr (ONE) column_one(j, width);
+        else good = column(j, width);
+    };
+    if constexpr (!ONE) {
+        T x[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) x[r] = a[r][0];
+        at_column(0);
+        candidate(0, x, [] {});
+        put_head();
+        send_row(std::integral_constant<int, NB>{});
     }
+    int j = 0;
+    if constexpr (NB == 64) {
+        for (; good && j < kmax && j < 16; ++j) run(j, std::integral_constant<int, 64>{});
+        for (; good && j < kmax && j < 32; ++j) run(j, std::integral_constant<int, 48>{});
+    }
+    if constexpr (NB >= 32)
+        for (; good && j < kmax && j < NB - 16; ++j) run(j, std::integral_constant<int, 32>{});
+    for (; good && j < kmax; ++j) run(j, std::integral_constant<int, 16>{});
+    __syncthreads();
+    // a row's entries are in its own thread's column of LDS (rows of U were
+    // written there by another wave, before the barrier)
 #pragma unroll
-    for (int r = 0; r < RPT; ++r) {
-        const int64_t i = base + (int64_t)r * NT;
-        if (i < m) {
-#pragma unroll
-            for (int c = 0; c < LEAF_COLS; ++c)
-                if (c < n) A[i + (int64_t)c * lda] = a[r][c];
+    for (int r = 0; r < R; ++r) {
+        const int i = first + t + r * NT;
+        if (i < m && good) {
+            const int q = pos[r] >= 0 ? pos[r] : -1 - pos[r];
+            T *row = A + q;
+            // live rows hold their columns of L and nothing past kmax; when
+            // kmax < n every row is a row of U
+            for (int c = 0; c < n; ++c) row[(int64_t)c * lda] = s_l[c][t + r * NT];
         }
     }
     if constexpr (ONE) return;
     __syncthreads();
     if (t == 0) {
         if (s_fail) st_agent(sync + SYNC_FLAG, 1);
-        // the last group out resets the counters (every group has passed
-        // every barrier by then)
-        const uint64_t prev = __hip_atomic_fetch_add(leave, (uint64_t)1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        // the last group out moves the tags on for the next launch (every
+        // group has read the epoch by then); near the end of the 32-bit range
+        // the recovery launch, alone on the stream, starts them over
+        const uint64_t prev = __hip_atomic_fetch_add(sync + SYNC_LEAVE, (uint64_t)1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
         if (prev == (uint64_t)G - 1) {
-            st_agent(arrive, 0);
-            st_agent(leave, 0);
+            st_agent(sync + SYNC_LEAVE, 0);
+            st_agent(sync + SYNC_EPOCH, (uint64_t)(epoch + (unsigned)NB));
         }
     }
 }
 
-// After every split leaf: nothing unless one of its waits ran out; then the
-// block saved before the leaf is put back, info restored, and the block
-// factored by the one-work-group global-memory leaf (pivots rewritten).
+// After every panel of several groups: nothing unless one of its waits ran
+// out; then the block saved before the panel is put back, info restored, and
+// the block factored by the one-work-group global-memory leaf (pivots
+// rewritten).  Tags near the end of their 32-bit range start over here, on
+// cleared slots, where no panel is running.
 template <typename T>
-__global__ __launch_bounds__(PIV_THREADS) void lu_leaf_recover_kernel(int64_t m, int n, T *__restrict__ A, int64_t lda,
-                                                                      int64_t *__restrict__ ipiv,
-                                                                      int64_t *__restrict__ info, int64_t r0,
-                                                                      uint64_t *__restrict__ sync) {
-    if (__hip_atomic_load(sync + SYNC_FLAG, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;
+__global__ __launch_bounds__(PIV_THREADS) void lu_panel_recover_kernel(int64_t m, int n, T *__restrict__ A, int64_t lda,
+                                                                       int64_t *__restrict__ ipiv,
+                                                                       int64_t *__restrict__ info, int64_t r0,
+                                                                       uint64_t *__restrict__ sync) {
+    const uint64_t flag = ld_agent(sync + SYNC_FLAG), epoch = ld_agent(sync + SYNC_EPOCH);
+    if (epoch > 0xf0000000u) {
+        __syncthreads();  // every wave has read the epoch
+        for (int i = threadIdx.x; i < SYNC_WORDS - SYNC_SLOTS; i += PIV_THREADS) st_agent(sync + SYNC_SLOTS + i, 0);
+        if (threadIdx.x == 0) st_agent(sync + SYNC_EPOCH, 0);
+    }
+    if (flag == 0) return;
     const T *save = reinterpret_cast<const T *>(sync + SYNC_WORDS);
     for (int64_t idx = threadIdx.x; idx < m * n; idx += PIV_THREADS) {
         const int64_t i = idx % m, c = idx / m;
-        A[i + c * lda] = save[i + c * SAVE_LD];
+        A[i + c * lda] = save[i + c * m];
     }
     if (threadIdx.x == 0) *info = (int64_t)sync[SYNC_INFO];
     __syncthreads();
@@ -627,17 +841,33 @@ struct LuRec {
     int64_t split_rows = lu_split_rows();
     int64_t spin_limit = lu_spin_limit() > 0 ? lu_spin_limit() : SPLIT_SPIN_LIMIT;
 
-    // an m x n leaf (n <= LEAF_COLS) over ceil(m / SPLIT_ROWS) work-groups
-    void split_leaf(int64_t m, int n, T *A, int64_t *ipiv, int64_t r0) {
+    template <int NB, int R, int NT>
+    void panel_of(int64_t m, int n, T *A, int64_t *ipiv, int64_t r0) {
+        const unsigned g = (unsigned)((m + NT * R - 1) / (NT * R));
+        if (g == 1) {
+            hipLaunchKernelGGL((lu_panel_kernel<T, NB, R, NT, true>), dim3(1), dim3(NT), 0, s, (int)m, n, A, lda, ipiv,
+                               info, r0, (uint64_t *)nullptr, (int64_t)0);
+            ok(hipGetLastError(), "lu panel");
+            return;
+        }
         uint64_t *sync = split_sync(s, &st);
         if (!sync) return;
-        const unsigned g = (unsigned)((m + SPLIT_ROWS - 1) / SPLIT_ROWS);
-        hipLaunchKernelGGL((lu_leaf_reg_kernel<T, SPLIT_THREADS, SPLIT_RPT, false>), dim3(g), dim3(SPLIT_THREADS), 0, s,
-                           m, n, A, lda, ipiv, info, r0, sync, spin_limit);
-        if (!ok(hipGetLastError(), "lu split leaf")) return;
-        hipLaunchKernelGGL(lu_leaf_recover_kernel<T>, dim3(1), dim3(PIV_THREADS), 0, s, m, n, A, lda, ipiv, info, r0,
+        hipLaunchKernelGGL((lu_panel_kernel<T, NB, R, NT, false>), dim3(g), dim3(NT), 0, s, (int)m, n, A, lda, ipiv,
+                           info, r0, sync, spin_limit);
+        if (!ok(hipGetLastError(), "lu panel")) return;
+        hipLaunchKernelGGL(lu_panel_recover_kernel<T>, dim3(1), dim3(PIV_THREADS), 0, s, m, n, A, lda, ipiv, info, r0,
                            sync);
-        ok(hipGetLastError(), "lu split leaf recovery");
+        ok(hipGetLastError(), "lu panel recovery");
+    }
+
+    // an m x n panel, n <= panel_cols(m): 128-row groups up to 8192 rows (each
+    // lane polls one group), 256 rows and more above
+    void panel(int64_t m, int n, T *A, int64_t *ipiv, int64_t r0) {
+        const int nb = panel_cols(m);
+        if (nb == 64 && m <= 8192) panel_of<64, 1, 128>(m, n, A, ipiv, r0);
+        else if (nb == 64) panel_of<64, 1, 256>(m, n, A, ipiv, r0);
+        else if (nb == 32) panel_of<32, 2, 256>(m, n, A, ipiv, r0);
+        else panel_of<16, 4, 256>(m, n, A, ipiv, r0);
     }
 
     bool ok(hipError_t e, const char *where) {
@@ -667,14 +897,9 @@ struct LuRec {
     // reference's "ipiv[i] += n1" (src/lu.jl:289-291) makes of them.
     void rec(int64_t m, int64_t n, T *A, int64_t *ipiv, int64_t r0) {
         if (st != NLA_OK || m == 0 || n == 0) return;
-        if (n <= LEAF_COLS && split_rows > 0 && m >= split_rows && m <= (int64_t)SPLIT_ROWS * SPLIT_MAX_WG) {
-            if (m <= ONE_ROWS) {
-                hipLaunchKernelGGL((lu_leaf_reg_kernel<T, ONE_THREADS, ONE_RPT, true>), dim3(1), dim3(ONE_THREADS), 0, s,
-                                   m, (int)n, A, lda, ipiv, info, r0, (uint64_t *)nullptr, (int64_t)0);
-                ok(hipGetLastError(), "lu register leaf");
-            } else {
-                split_leaf(m, (int)n, A, ipiv, r0);
-            }
+        const int nb = split_rows > 0 && m >= split_rows ? panel_cols(m) : 0;
+        if (n <= nb) {
+            panel(m, (int)n, A, ipiv, r0);
             return;
         }
         if (n <= LEAF_COLS || m == 1) {
@@ -683,7 +908,10 @@ struct LuRec {
             ok(hipGetLastError(), "lu leaf");
             return;
         }
-        const int64_t mn = m < n ? m : n, n1 = mn / 2, n2 = n - n1;
+        // whole panels on the left: n1 is half of the columns rounded up to a
+        // multiple of the panel's width (all of a block of at most nb rows)
+        const int64_t mn = m < n ? m : n, half = nb > 0 ? ((mn + 1) / 2 + nb - 1) / nb * nb : mn / 2;
+        const int64_t n1 = half < mn ? half : (mn < n ? mn : mn / 2), n2 = n - n1;
         rec(m, n1, A, ipiv, r0);
         laswp(A + n1 * lda, m, n2, 1, n1, ipiv, r0);
         if (st != NLA_OK) return;
@@ -700,7 +928,8 @@ struct LuRec {
             }
         }
         // A22 -= A21 A12
-        if (m > n1) {
+        if (m <= n1) return;
+        {
             const int32_t r = nla_gemm(dtype, 'N', 'N', m - n1, n2, n1, -1.0, A + n1, lda, A + n1 * lda, lda, 1.0,
                                        A + n1 + n1 * lda, lda, s);
             if (r != NLA_OK) {

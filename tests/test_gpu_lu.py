@@ -231,3 +231,26 @@ def test_split_leaf_timeout_is_recovered(nla, split_rows, spin_limit, m, n):
     spin_limit(0)
     L3, p3, i3 = nla.getrf2_(A0.clone())  # and the normal path after a recovery
     assert i3 == 4 and torch.equal(p1, p3) and torch.equal(L1, L3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("m,n", [(33, 64), (128, 64), (129, 65), (257, 63), (8192, 17), (8193, 64), (32769, 33),
+                                 (65537, 17)])
+def test_register_panel_edges(nla, split_rows, dtype, m, n):
+    """Panels at the edges of their groups (128 rows, 256 above 8192) and
+    column counts (64, 32 above 32768 rows, 16 above 65536), wide and with a
+    column more than the panel takes: the pivots and the factors of the
+    global-memory leaf, with equal entries in a column (ties go to the first
+    row) among the inputs."""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(3 * m + n)
+    A0 = torch.empty((n, m), dtype=dtype, device=DEV).normal_(generator=g).t()
+    A0[:, 0] = 1.0  # every row ties for the first pivot
+    split_rows(0)
+    L1, p1, i1 = nla.getrf2_(A0.clone())
+    split_rows(1)
+    L2, p2, i2 = nla.getrf2_(A0.clone())
+    assert i1 == i2 == 0 and p1[0].item() == 1
+    assert torch.equal(p1, p2)
+    tol = 1e-12 if dtype == torch.float64 else 1e-5
+    assert torch.max(torch.abs(L1 - L2)).item() <= tol * torch.max(torch.abs(L1)).item()
