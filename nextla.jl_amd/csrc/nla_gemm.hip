@@ -472,7 +472,7 @@ static hipError_t launch_tri_dense(const GemmArgs<T> &a, hipStream_t s) {
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 template <typename T>
-hipError_t launch_gemm(const GemmArgs<T> &a, hipStream_t s) {
+hipError_t launch_gemm_tiled(const GemmArgs<T> &a, hipStream_t s) {
     if (a.M <= 0 || a.N <= 0) return hipSuccess;
     constexpr int VW = 16 / sizeof(T);
     // 16-byte vector loads need every column start of X, Y (and the tile
@@ -626,7 +626,7 @@ template hipError_t launch_grouped_gemm<float>(const GroupGemm<float> *, const i
 template hipError_t launch_grouped_gemm<double>(const GroupGemm<double> *, const int2 *, int, int *, bool, bool,
                                                 bool, bool, bool, int, hipStream_t);
 
-template hipError_t launch_gemm<float>(const GemmArgs<float> &, hipStream_t);
-template hipError_t launch_gemm<double>(const GemmArgs<double> &, hipStream_t);
+template hipError_t launch_gemm_tiled<float>(const GemmArgs<float> &, hipStream_t);
+template hipError_t launch_gemm_tiled<double>(const GemmArgs<double> &, hipStream_t);
 
 }  // namespace nla

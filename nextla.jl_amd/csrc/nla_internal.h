@@ -195,8 +195,12 @@ hipError_t launch_batch(const BatchSys<T> *sys, const BatchTask *tasks, int ntas
 template <typename T>
 hipError_t launch_batch_trtri(const BatchSys<T> *sys, const int2 *blk, int nblk, hipStream_t s);
 
+// The product by the kernel that suits its shape: the tiled kernels, or the
+// K-splitting one where their tiles would leave most of the chip idle.
 template <typename T>
 hipError_t launch_gemm(const GemmArgs<T> &a, hipStream_t s);
+template <typename T>
+hipError_t launch_gemm_tiled(const GemmArgs<T> &a, hipStream_t s);
 
 template <typename T>
 hipError_t launch_leaf(const LeafArgs<T> &a, hipStream_t s);
