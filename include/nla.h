@@ -571,8 +571,9 @@ int32_t nla_serve_destroy(nla_server server);
  *   NLA_CFG_PANEL_STRIP_F32 / _F64: right-hand-side columns per panel
  *                      work-group, 16 (default) or 32;
  *   NLA_CFG_PANEL_WAVES: waves per panel work-group (panels up to 512 rows):
- *                      4, or 8, where two waves share each 16-row output
- *                      tile and split its k range; 0 (default) = 4;
+ *                      4 (left-looking, 16 columns, two and more groups per
+ *                      CU) or 8 (32-row units, right-looking TRSM); 0
+ *                      (default) by the panel's rows and columns;
  *   NLA_CFG_BATCH_CLASSES: size classes new batch plans may use, bit c for
  *                      systems up to 128 << c rows (c = 0..3; the 1024 class
  *                      is always on; default 0x1F: all, with bit 4).  A system goes to the

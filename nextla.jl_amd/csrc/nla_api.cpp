@@ -123,11 +123,7 @@ static std::atomic<int> g_panel{-1};
 static std::atomic<int> g_panel_rows[2] = {{0}, {0}};
 static int panel_rows_default(bool contiguous) { return contiguous ? 512 : 256; }
 static std::atomic<int> g_panel_strip[2] = {{PANEL_STRIP}, {PANEL_STRIP}};
-// Waves per panel work-group: 0 = the default, 4 (measured on MI355X at
-// n = 8192 with 512-row panels: 4 waves against 8, which split each phase's
-// k range, FP32 TRSM 4.83 / 4.95 ms, FP32 TRMM 4.80 / 4.87, FP64 TRMM
-// 9.03 / 9.10, FP64 TRSM 9.36 / 9.62, the refined solve's fp32 panels
-// 33.1 / 33.5 ms), else 4 or 8 for every panel.
+// Waves per panel work-group: 4, 8, or 0 = by the panel's shape (launch_panel).
 static std::atomic<int> g_panel_waves{0};
 // Batch size classes: all four, systems above 512 rows staged (measured on
 // MI355X over 10,000 systems of 16..1024 rows: 5.5 ms vs 6.9 ms with
@@ -198,7 +194,7 @@ struct Recursion {
     const int *F = nullptr; // their ill-conditioning flags (refined in the panels)
     int mode = 1;
     bool use_panel = true;  // fuse diagonal blocks <= panel_rows into one launch
-    int panel_rows = 512, panel_strip = PANEL_STRIP, panel_waves = 4;
+    int panel_rows = 512, panel_strip = PANEL_STRIP, panel_waves = 0;
     bool unit = false;  // unit diagonal: only the panels and the inverses read the diagonal
     hipError_t err = hipSuccess;
     // Low-precision GEMM updates (T = float only): lp = 0 bf16, 1 fp16,
@@ -279,7 +275,7 @@ struct Recursion {
             a.wrs = nb; a.wcs = 1;
         }
         a.strip = panel_strip;
-        a.waves = n <= 512 ? panel_waves : 4;
+        a.waves = panel_waves;
         a.unit = unit;
         if constexpr (sizeof(T) == 4) {
             if (x_slots && func == 'S') a.xmax = x_slots + off / 64;
@@ -550,8 +546,7 @@ static int32_t rectrxm_typed(char side, char uplo, char trans, char func, double
         const bool contiguous = (side == 'L' ? A.rs : A.cs) == 1;
         r.panel_rows = pr ? pr : panel_rows_default(contiguous);
         r.panel_strip = g_panel_strip[di].load();
-        const int pw = g_panel_waves.load();
-        r.panel_waves = pw ? pw : 4;
+        r.panel_waves = g_panel_waves.load();
     }
     T *W = nullptr;
     std::unique_lock<std::mutex> hold;
@@ -779,7 +774,7 @@ static int32_t rectrxm_mixed_impl(char side, char uplo, char trans, int precisio
         r.use_panel = true;
         r.W = W;
         r.F = WF;
-        r.panel_waves = g_panel_waves.load() ? g_panel_waves.load() : 4;
+        r.panel_waves = g_panel_waves.load();
         const bool scaled = (prec == NLA_LP_FP16 || prec == NLA_LP_FP16X2);
         if (prec != NLA_LP_FP32) r.lp = (prec == NLA_LP_FP16X2) ? 2 : prec;
         if (scaled) {

@@ -77,7 +77,7 @@ struct PanelArgs {
     const int *F = nullptr;
     int strip = PANEL_STRIP;  // RHS columns per work-group: 16 or 32
     bool unit = false;        // unit diagonal (taken as 1, not read)
-    int waves = 4;            // waves per work-group: 4, or 8 splitting each phase's k range (<= 512 rows)
+    int waves = 0;            // waves per work-group up to 512 rows: 4, 8, or 0 by shape
     // TRSM, fp32: *xmax = max(*xmax, max |X|) over the panel's solution (a
     // float bit pattern), the scale source of the updates that read it
     unsigned *xmax = nullptr;

@@ -119,12 +119,9 @@ __device__ inline int phase_count(int nsb, bool trmm) {
 }
 
 // Solve / multiply one strip of W columns (starting at c0) of one diagonal
-// panel; bs is the LDS strip (W x LDB).  NW waves: with 4, wave w computes
-// rows 16w..16w+15 of every 64-row phase over its whole 64-deep k range;
-// with 8, waves w and w+4 share those rows and take one half of the k range
-// each (twice the waves to hide latency with the same work), their partial
-// sums meeting in the 64 x W LDS scratch sc when a block is written.
-template <typename T, int NBIG, int WS, bool TRMM, int NW = 4>
+// panel; bs is the LDS strip (W x LDB).  Four waves: wave w computes rows
+// 16w..16w+15 of every 64-row phase over its 64-deep k range.
+template <typename T, int NBIG, int WS, bool TRMM>
 // Always inlined: with the single-panel kernel and the batched kernel both
 // calling one instantiation, the compiler otherwise emits a real call (and
 // the panel ran 50 % slower).
@@ -139,10 +136,9 @@ __device__ __forceinline__ void panel_strip(int nbig, int64_t m, int64_t c0, con
     constexpr int W = PS::W;
     constexpr int LDB = NBIG + (sizeof(T) == 8 ? 2 : 4);
     constexpr int NKS = 64 / MF::KD;  // k-steps per 64-deep phase
-    static_assert(NW == 4 || NW == 8, "4 or 8 waves");
-    constexpr int NT = NW * 64, KSPLIT = NW / 4, NKW = NKS / KSPLIT;  // k-steps per wave
+    constexpr int NW = 4, NT = NW * 64, NKW = NKS;
 
-    const int t = threadIdx.x, lane = t & 63, wave = (t >> 6) & 3, kh = (t >> 6) >> 2;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int nsb = (nbig + 63) / 64;
 
     // ---- load the strip (coalesced along B's contiguous direction) ----
@@ -208,7 +204,7 @@ __device__ __forceinline__ void panel_strip(int nbig, int64_t m, int64_t c0, con
     // as a bit mask.
     static_assert(MF::KD == 4, "four k per MFMA step");
     const int fi = rb * MF::BD + lo;            // the lane's row of a block
-    const int kb = kh * NKW * MF::KD + lk;      // the lane's first k
+    const int kb = lk;                          // the lane's first k
     auto span = [](int c) { return c <= 0 ? 0u : (c >= NKW ? (NKW >= 32 ? ~0u : (1u << NKW) - 1u) : (1u << c) - 1u); };
     // global address space spelled out: a select between the block and
     // panel_zero otherwise degrades the loads to flat ones; its address is
@@ -263,7 +259,7 @@ __device__ __forceinline__ void panel_strip(int nbig, int64_t m, int64_t c0, con
         for (int sw = 0; sw < NKW; ++sw)
 #pragma unroll
             for (int cb = 0; cb < PS::CBW; ++cb)
-                bv[sw][cb] = src[((cbase + cb) * MF::BD + lo) * LDB + (kh * NKW + sw) * MF::KD + lk];
+                bv[sw][cb] = src[((cbase + cb) * MF::BD + lo) * LDB + sw * MF::KD + lk];
         // keep the scheduler from sinking the reads back next to their MFMAs
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(1);  // issue priority while in the MFMA cluster
@@ -280,32 +276,6 @@ __device__ __forceinline__ void panel_strip(int nbig, int64_t m, int64_t c0, con
     };
     auto write_block = [&](int ib, T alpha, T beta) {
         NLA_LDS T *dst = bs + ib * 64;
-        if constexpr (KSPLIT == 2) {
-            // the second k half hands its partial sums to the first
-            if (kh == 1) {
-#pragma unroll
-                for (int cb = 0; cb < PS::CBW; ++cb)
-#pragma unroll
-                    for (int r = 0; r < MF::NR; ++r) {
-                        const int row = rb * MF::BD + MF::di(lane, r);
-                        const int col = (cbase + cb) * MF::BD + MF::dj(lane, r);
-                        sc[col * 64 + row] = acc[cb][r] + acc2[cb][r];
-                    }
-            }
-            __syncthreads();
-            if (kh == 1) return;
-#pragma unroll
-            for (int cb = 0; cb < PS::CBW; ++cb)
-#pragma unroll
-                for (int r = 0; r < MF::NR; ++r) {
-                    const int row = rb * MF::BD + MF::di(lane, r);
-                    const int col = (cbase + cb) * MF::BD + MF::dj(lane, r);
-                    NLA_LDS T *p = dst + col * LDB + row;
-                    T v = alpha * ((acc[cb][r] + acc2[cb][r]) + sc[col * 64 + row]);
-                    *p = (beta == T(0)) ? v : v + beta * *p;
-                }
-            return;
-        }
 #pragma unroll
         for (int cb = 0; cb < PS::CBW; ++cb)
 #pragma unroll
@@ -490,54 +460,651 @@ __device__ __forceinline__ void panel_strip(int nbig, int64_t m, int64_t c0, con
     }
 }
 
-template <typename T, int NBIG, int WS, bool TRMM, int NW>
-__global__ __launch_bounds__(NW * 64) void panel_kernel(int nbig, int64_t m, const T *__restrict__ Mp, int64_t mrs,
-                                                        int64_t mcs, int lower, int unit, T *__restrict__ Bp,
-                                                        int64_t brs, int64_t bcs, const T *__restrict__ Wp,
-                                                        int64_t wrs, int64_t wcs, T scale,
-                                                        const int *__restrict__ Fp, unsigned *xmax) {
+// The left-looking strip of the batched solver as one launch: for panels with
+// little of a chain or more strips than compute units (below), and above 512
+// rows (taken only when a larger panel size is set).
+template <typename T, int NBIG, int WS, bool TRMM>
+__global__ __launch_bounds__(256) void panel_left_kernel(int nbig, int64_t m, const T *__restrict__ Mp,
+                                                             int64_t mrs, int64_t mcs, int lower, int unit,
+                                                             T *__restrict__ Bp, int64_t brs, int64_t bcs,
+                                                             const T *__restrict__ Wp, int64_t wrs, int64_t wcs,
+                                                             T scale, const int *__restrict__ Fp, unsigned *xmax) {
     constexpr int LDB = NBIG + (sizeof(T) == 8 ? 2 : 4);
     __shared__ __attribute__((aligned(16))) T bs_raw[WS * LDB];
-    // k-split partial sums (8 waves) and the refinement step's scratch
-    __shared__ __attribute__((aligned(16))) T sc_raw[(NW == 8 || !TRMM) ? 64 * WS : 1];
-    panel_strip<T, NBIG, WS, TRMM, NW>(nbig, m, (int64_t)blockIdx.x * WS, Mp, mrs, mcs, lower != 0, unit != 0, Bp,
+    // the refinement step's scratch
+    __shared__ __attribute__((aligned(16))) T sc_raw[!TRMM ? 64 * WS : 1];
+    panel_strip<T, NBIG, WS, TRMM>(nbig, m, (int64_t)blockIdx.x * WS, Mp, mrs, mcs, lower != 0, unit != 0, Bp,
                                        brs, bcs, Wp, wrs, wcs, scale, Fp, (NLA_LDS T *)bs_raw,
                                        (NLA_LDS T *)sc_raw, xmax);
 }
 
-template <typename T, int NBIG, int W, int NW>
-static hipError_t launch_panel_w(const PanelArgs<T> &a, hipStream_t s) {
-    const int64_t groups = (a.m + W - 1) / W;
+// ---------------------------------------------------------------------------
+// Panels of up to 512 rows: a work-group of eight waves per strip of W
+// columns, the strip in LDS.
+//
+// What bounds a panel: with few strips the chain of diagonal blocks, with
+// many the matrix cores, and in between the rate at which a CU's address
+// unit takes load instructions (16 cycles each whatever their width: with one
+// element per lane the M operand's loads took as long as its FP64 MFMAs, and
+// twice as long in FP32).  So:
+//   - the rows are dealt out in units of 32, two MFMA row blocks, and a lane
+//     loads the two rows 2l, 2l + 1 of a column of M at once, or four
+//     consecutive k where M is contiguous along k (KC);
+//   - TRSM runs right-looking.  A wave owns units w and w + 8 (in solving
+//     order) and keeps sum M_ik X_k of each in its accumulators, apart from
+//     B as the left-looking order does, so nothing of its precision is lost;
+//     a step subtracts the sums of one 64-block from B, multiplies by the
+//     inverse (four waves) and then all waves add the new block's products
+//     to every unit still owed at once.  Two barriers per 64-block;
+//   - a 32-deep piece of M is always on its way while the one before it is
+//     used.  The loops have no load under a branch (the compiler would wait
+//     at the join): a wave's steps are split by which of its units are still
+//     active, and the waves that apply the inverse run their own copy;
+//   - TRMM has no chain: every wave forms units w and 15 - w, whose parts of
+//     the triangle add up to the same, from the strip in LDS.
+
+template <typename T>
+struct Mat2 {
+    typedef T v2_t __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+    typedef T v4_t __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+};
+
+constexpr int PU_WAVES = 8, PU_MAX = 512;
+
+// One unit's rows of M: row block b of the unit holds rows 2l + b (l = lane %
+// 16), or 16 b + l where M is contiguous along k.
+template <typename T, bool KC>
+struct PanelRows {
+    const T *p[KC ? 2 : 1];  // the lane's row(s), at its k = 4 (lane / 16)
+    int64_t cs;
+    __device__ static inline int row(int b, int lo) { return KC ? 16 * b + lo : 2 * lo + b; }
+    // r0: the unit's first row; rows past the panel read its last row (an
+    // even row's pair may reach one element past it, which is the next column
+    // of a matrix that has one: off the diagonal k + 1 < nbig)
+    __device__ inline void init(const T *M, int64_t mrs, int64_t mcs, int r0, int nbig, int lane) {
+        const int lo = lane & 15, kk = 4 * (lane >> 4);
+        cs = mcs;
+#pragma unroll
+        for (int b = 0; b < (KC ? 2 : 1); ++b) {
+            const int r = r0 + row(b, lo);
+            p[b] = M + (int64_t)(r < nbig ? r : nbig - 1) * mrs + (int64_t)kk * mcs;
+        }
+    }
+    // f[b][4 q + e] = M(row b, k0 + 16 q + kk + e), q < 2
+    __device__ inline void load(int k0, T (*f)[8]) const {
+        if constexpr (KC) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    if constexpr (sizeof(T) == 8) {
+                        const typename Mat2<T>::v2_t x = *(const typename Mat2<T>::v2_t *)(p[b] + k0 + 16 * q);
+                        const typename Mat2<T>::v2_t y = *(const typename Mat2<T>::v2_t *)(p[b] + k0 + 16 * q + 2);
+                        f[b][4 * q] = x[0];
+                        f[b][4 * q + 1] = x[1];
+                        f[b][4 * q + 2] = y[0];
+                        f[b][4 * q + 3] = y[1];
+                    } else {
+                        const typename Mat2<T>::v4_t x = *(const typename Mat2<T>::v4_t *)(p[b] + k0 + 16 * q);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) f[b][4 * q + e] = x[e];
+                    }
+                }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const typename Mat2<T>::v2_t x =
+                        *(const typename Mat2<T>::v2_t *)(p[0] + (int64_t)(k0 + 16 * q + e) * cs);
+                    f[0][4 * q + e] = x[0];
+                    f[1][4 * q + e] = x[1];
+                }
+        }
+    }
+};
+
+// The same element by element, zero (and not read) outside [lo_k, hi_k) of
+// its row: M(r, k0 + ...) with r the row block's row.
+template <typename T>
+__device__ __forceinline__ void panel_masked(const T *__restrict__ M, int64_t mrs, int64_t mcs, int r, int k0, int ka,
+                                             int kb, int lane, T *f) {
+    // global address space spelled out: a select between the block and
+    // panel_zero otherwise degrades the loads to flat ones
+    typedef const __attribute__((address_space(1))) T GT;
+    GT *zp = (GT *)panel_zero;
+    const int kk = 4 * (lane >> 4);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int k = k0 + 16 * q + kk + e;
+            f[4 * q + e] = *(k >= ka && k < kb ? (GT *)(M + (int64_t)r * mrs + (int64_t)k * mcs) : zp);
+        }
+}
+
+// Sums of NB row blocks, in two sets (even and odd k of a lane): two
+// independent MFMA chains, and sums half as long to round.
+template <typename T, int NB, int CBW>
+struct PanelAcc {
+    typedef Mfma16<T> MF;
+    typename MF::acc_t a[2][NB][CBW];
+    __device__ inline void zero() {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int cb = 0; cb < CBW; ++cb) a[i][b][cb] = MF::zero();
+    }
+    __device__ inline T at(int b, int cb, int e) const { return a[0][b][cb][e] + a[1][b][cb][e]; }
+};
+
+// acc += f (32 deep) times x: xs points at the lane's column and its first k
+// in LDS, column blocks 16 * ldx apart.
+template <typename T, int CBW, int NB>
+__device__ __forceinline__ void panel_mul(const T (*f)[8], const NLA_LDS T *xs, int ldx,
+                                          PanelAcc<T, NB, CBW> &acc) {
+    typedef Mfma16<T> MF;
+    T x[CBW][8];
+#pragma unroll
+    for (int cb = 0; cb < CBW; ++cb)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[cb][4 * q + e] = xs[cb * 16 * ldx + 16 * q + e];
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int cb = 0; cb < CBW; ++cb)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) acc.a[e & 1][b][cb] = MF::mma(x[cb][e], f[b][e], acc.a[e & 1][b][cb]);
+    __builtin_amdgcn_s_setprio(0);
+}
+
+template <typename T>
+constexpr int panel_pad() {
+    return 16 / (int)sizeof(T);  // 16-byte LDS reads of 16 columns start in different banks
+}
+
+// The strip between B and LDS, along B's contiguous direction, loads in
+// batches so that their latencies overlap; rows past the panel and columns
+// past m are zero in LDS.
+template <typename T, int W, int LDB>
+__device__ __forceinline__ void panel_load(const T *__restrict__ Bp, int64_t brs, int64_t bcs, int nbig, int nrow,
+                                           int64_t ncol, T scale, NLA_LDS T *bs) {
+    constexpr int NT = PU_WAVES * 64;
+    const int t = threadIdx.x;
+    if (brs == 1) {
+        for (int r = t; r < nrow; r += NT) {
+            T v[W];
+#pragma unroll
+            for (int c = 0; c < W; ++c) {
+                const bool ok = r < nbig && c < ncol;
+                v[c] = *(ok ? Bp + r + c * bcs : Bp);
+                v[c] = ok ? v[c] * scale : T(0);
+            }
+#pragma unroll
+            for (int c = 0; c < W; ++c) bs[c * LDB + r] = v[c];
+        }
+    } else {
+        const int c = t % W;
+        const bool cok = c < ncol;
+        constexpr int SL = 8, RSTEP = NT / W;
+        for (int r0 = t / W; r0 < nrow; r0 += RSTEP * SL) {
+            T v[SL];
+#pragma unroll
+            for (int u = 0; u < SL; ++u) {
+                const int r = r0 + u * RSTEP;
+                const bool ok = cok && r < nbig;
+                v[u] = *(ok ? Bp + r * brs + c * bcs : Bp);
+                v[u] = ok ? v[u] * scale : T(0);
+            }
+#pragma unroll
+            for (int u = 0; u < SL; ++u)
+                if (r0 + u * RSTEP < nrow) bs[c * LDB + r0 + u * RSTEP] = v[u];
+        }
+    }
+}
+
+template <typename T, int W, int LDB>
+__device__ __forceinline__ T panel_store(T *__restrict__ Bp, int64_t brs, int64_t bcs, int nbig, int64_t ncol,
+                                         const NLA_LDS T *bs) {
+    constexpr int NT = PU_WAVES * 64;
+    const int t = threadIdx.x;
+    T vmax = T(0);  // a NaN compares false and never raises it
+    if (brs == 1) {
+        for (int r = t; r < nbig; r += NT) {
+#pragma unroll
+            for (int c = 0; c < W; ++c) {
+                const T v = bs[c * LDB + r];
+                if (c < ncol) {
+                    Bp[r + c * bcs] = v;
+                    vmax = fabs(v) > vmax ? fabs(v) : vmax;
+                }
+            }
+        }
+    } else {
+        const int c = t % W;
+        if (c < ncol) {
+            for (int r = t / W; r < nbig; r += NT / W) {
+                const T v = bs[c * LDB + r];
+                Bp[r * brs + c * bcs] = v;
+                vmax = fabs(v) > vmax ? fabs(v) : vmax;
+            }
+        }
+    }
+    return vmax;
+}
+
+// One strip's TRSM.  bs: the strip (W x LDB), tmp: a 64 x W block.
+template <typename T, int W, int LDB, bool KC>
+struct PanelSolve {
+    typedef Mfma16<T> MF;
+    typedef PanelRows<T, KC> PR;
+    static constexpr int CBW = W / 16, LDX = 64 + panel_pad<T>();
+    typedef PanelAcc<T, 1, CBW> X;  // a row block of X
+    int nbig, nsb, lane, wv, lo, kk;
+    bool lower, unit;
+    const T *Mp;
+    int64_t mrs, mcs;
+    const T *Wp;
+    int64_t wrs, wcs;
+    const int *Fp;
+    NLA_LDS T *bs, *tmp;
+    PR rows[2];
+    PanelAcc<T, 2, CBW> acc[2];
+    T fw[16];
+
+    __device__ inline int block(int s) const { return lower ? s : nsb - 1 - s; }
+    // first row of the j-th unit of this wave (in solving order)
+    __device__ inline int unit_row(int j) const {
+        const int u = wv + PU_WAVES * j;
+        return 64 * block(u >> 1) + 32 * (u & 1);
+    }
+    __device__ inline void load_inverse(int s) {
+        const T *p = Wp + (int64_t)block(s < nsb ? s : nsb - 1) * 64 * 64 + (16 * wv + lo) * wrs + kk * wcs;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) fw[4 * q + e] = p[(16 * q + e) * wcs];
+    }
+    __device__ inline int k_of(int s, int h) const { return 64 * block(s) + 32 * h; }
+
+    // tmp = B_s - (the sums of unit j)
+    __device__ inline void put(int j) {
+        const int r0 = unit_row(j), b0 = r0 & 63;
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int cb = 0; cb < CBW; ++cb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int c = cb * 16 + MF::di(lane, e), i = PR::row(b, lo);
+                    const T v = bs[c * LDB + r0 + i] - acc[j].at(b, cb, e);
+                    tmp[c * LDX + b0 + i] = r0 + i < nbig ? v : T(0);
+                }
+    }
+    // x (+)= the inverse's row block times tmp
+    __device__ inline void apply_inverse(X &x) {
+        T g[1][8];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) g[0][e] = fw[8 * h + e];
+            panel_mul<T, CBW, 1>(g, tmp + lo * LDX + 32 * h + kk, LDX, x);
+        }
+    }
+    __device__ inline void put_x(int s, const X &x) {
+        const int r0 = 64 * block(s) + 16 * wv + lo;
+#pragma unroll
+        for (int cb = 0; cb < CBW; ++cb)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                bs[(cb * 16 + MF::di(lane, e)) * LDB + r0] = r0 < nbig ? x.at(0, cb, e) : T(0);
+    }
+    // An ill-conditioned diagonal block: X += inv(M_ss) (B_s - M_ss X).  A
+    // rare path; every wave passes its barriers.
+    template <bool DIAG>
+    __device__ inline void refine(int s, X &x) {
+        const int bl = block(s), nb = bl == nsb - 1 ? nbig - 64 * bl : 64, i = 16 * wv + lo, r = 64 * bl + i;
+        X v;
+        T res[CBW][4];
+        if (DIAG) put_x(s, x);
+        __syncthreads();
+        if (DIAG) {
+            v.zero();
+            const int ka = lower ? 0 : (unit ? i + 1 : i), kb = i < nb ? (lower ? (unit ? i : i + 1) : nb) : 0;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                T g[1][8];
+                panel_masked<T>(Mp, mrs, mcs, i < nb ? r : nbig - 1, 64 * bl + 32 * h, 64 * bl + ka, 64 * bl + kb, lane,
+                                g[0]);
+                panel_mul<T, CBW, 1>(g, bs + lo * LDB + 64 * bl + 32 * h + kk, LDB, v);
+            }
+#pragma unroll
+            for (int cb = 0; cb < CBW; ++cb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int c = cb * 16 + MF::di(lane, e);
+                    const T mx = unit && i < nb ? v.at(0, cb, e) + x.at(0, cb, e) : v.at(0, cb, e);
+                    res[cb][e] = tmp[c * LDX + i] - mx;
+                }
+        }
+        __syncthreads();
+        if (DIAG) {
+#pragma unroll
+            for (int cb = 0; cb < CBW; ++cb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    tmp[(cb * 16 + MF::di(lane, e)) * LDX + i] = i < nb ? res[cb][e] : T(0);
+        }
+        __syncthreads();
+        if (DIAG) apply_inverse(x);
+    }
+    // Solves block s into the strip: sums out, inverse, X in; two barriers.
+    template <bool DIAG>
+    __device__ inline void diagonal(int s) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            if (((wv + PU_WAVES * j) >> 1) == s) put(j);
+        __syncthreads();
+        X x;
+        if (DIAG) {
+            x.zero();
+            apply_inverse(x);
+        }
+        if (Fp != nullptr && Fp[block(s)] != 0) refine<DIAG>(s, x);
+        if (DIAG) put_x(s, x);
+        __syncthreads();
+        if (DIAG) load_inverse(s + 1);
+    }
+    // Steps [s0, s1) with units 0 and / or 1 of this wave still owed.
+    template <bool DIAG, bool U0, bool U1>
+    __device__ inline void steps(int s0, int s1) {
+        if (s0 >= s1) return;
+        T f[2][2][8];
+        constexpr int J = U0 ? 0 : 1;
+        if constexpr (U0 || U1) {
+            rows[J].load(k_of(s0, 0), f[0]);
+            rows[J].load(k_of(s0, 1), f[1]);
+        }
+        for (int s = s0; s < s1; ++s) {
+            diagonal<DIAG>(s);
+            const int sn = s + 1 < s1 ? s + 1 : s;  // past the last step, this block again
+            const NLA_LDS T *xs = bs + lo * LDB + k_of(s, 0) + kk;
+            if constexpr (U0 || U1) {
+                panel_mul<T, CBW, 2>(f[0], xs, LDB, acc[J]);
+                rows[U0 && U1 ? 1 : J].load(k_of(U0 && U1 ? s : sn, 0), f[0]);
+                panel_mul<T, CBW, 2>(f[1], xs + 32, LDB, acc[J]);
+                rows[U0 && U1 ? 1 : J].load(k_of(U0 && U1 ? s : sn, 1), f[1]);
+            }
+            if constexpr (U0 && U1) {
+                panel_mul<T, CBW, 2>(f[0], xs, LDB, acc[1]);
+                rows[0].load(k_of(sn, 0), f[0]);
+                panel_mul<T, CBW, 2>(f[1], xs + 32, LDB, acc[1]);
+                rows[0].load(k_of(sn, 1), f[1]);
+            }
+        }
+    }
+    // The first step of an upper panel whose last block is short: its k range
+    // ends inside a 64-block.
+    template <bool DIAG>
+    __device__ inline void short_step() {
+        diagonal<DIAG>(0);
+        const int k0 = 64 * (nsb - 1);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int u = wv + PU_WAVES * j;
+            if (u < 2 || u >= 2 * nsb) continue;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                T f[2][8];
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    panel_masked<T>(Mp, mrs, mcs, unit_row(j) + PR::row(b, lo), k0 + 32 * h, 0, nbig, lane, f[b]);
+                panel_mul<T, CBW, 2>(f, bs + lo * LDB + k0 + 32 * h + kk, LDB, acc[j]);
+            }
+        }
+    }
+    template <bool DIAG>
+    __device__ inline void run() {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if (wv + PU_WAVES * j < 2 * nsb) rows[j].init(Mp, mrs, mcs, unit_row(j), nbig, lane);
+            else rows[j].init(Mp, mrs, mcs, 0, nbig, lane);
+            acc[j].zero();
+        }
+        if (DIAG) load_inverse(0);
+        int s = 0;
+        if (!lower && (nbig & 63) != 0) {
+            short_step<DIAG>();
+            s = 1;
+        }
+        const int n0 = wv < 2 * nsb ? wv >> 1 : 0, n1 = wv + PU_WAVES < 2 * nsb ? (wv + PU_WAVES) >> 1 : 0;
+        auto later = [&](int n) { return n > s ? n : s; };
+        if (n1 > 0) {
+            steps<DIAG, true, true>(s, n0);
+            s = later(n0);
+            steps<DIAG, false, true>(s, n1);
+            s = later(n1);
+        } else {
+            steps<DIAG, true, false>(s, n0);
+            s = later(n0);
+        }
+        steps<DIAG, false, false>(s, nsb);
+        __syncthreads();
+    }
+};
+
+template <typename T, int NBIG, int W, bool KC>
+__device__ __forceinline__ void panel_trmm(int nbig, int64_t m, int64_t c0, const T *__restrict__ Mp, int64_t mrs,
+                                           int64_t mcs, bool lower, bool unit, T *__restrict__ Bp, int64_t brs,
+                                           int64_t bcs, T scale, NLA_LDS T *bs) {
+    typedef Mfma16<T> MF;
+    typedef PanelRows<T, KC> PR;
+    constexpr int CBW = W / 16, LDB = NBIG + panel_pad<T>(), PD = 3;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int lo = lane & 15, kk = 4 * (lane >> 4);
+    const int64_t ncol = m - c0 < W ? m - c0 : W;
+    T *B = Bp + c0 * bcs;
+    panel_load<T, W, LDB>(B, brs, bcs, nbig, (nbig + 31) / 32 * 32, ncol, T(1), bs);
+    __syncthreads();
+    const int nu = (nbig + 31) / 32;
+    const NLA_LDS T *xb = bs + lo * LDB + kk;
+    for (int j = 0; j < 2; ++j) {
+        // units w and 2 nw - 1 - w of the nu: parts of the triangle that add up alike
+        const int u = j == 0 ? wv : 2 * PU_WAVES - 1 - wv;
+        if (u >= nu) continue;
+        const int r0 = 32 * u;
+        PanelAcc<T, 2, CBW> acc;
+        acc.zero();
+        // off the diagonal, whole 32-deep pieces: [ka, kb); an upper unit's last one may be short
+        const int ka = lower ? 0 : r0 + 32, kb = lower ? r0 : nbig, np = (kb - ka) / 32;
+        PR rows;
+        rows.init(Mp, mrs, mcs, r0, nbig, lane);
+        T f[PD][2][8], d[2][8];
+        if (np > 0) {
+#pragma unroll
+            for (int v = 0; v < PD - 1; ++v) rows.load(ka + 32 * (v < np ? v : np - 1), f[v]);
+        }
+        // the diagonal piece, masked to the triangle (what a whole piece reads
+        // beside it is dropped, whatever it holds)
+        const bool whole = r0 + 32 <= nbig;
+        if (whole) rows.load(r0, d);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int r = r0 + PR::row(b, lo);
+            const int k0 = lower ? r0 : (unit ? r + 1 : r), k1 = lower ? (unit ? r : r + 1) : nbig;
+            if (!whole) {
+                panel_masked<T>(Mp, mrs, mcs, r < nbig ? r : nbig - 1, r0, k0, r < nbig ? k1 : 0, lane, d[b]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int k = r0 + 16 * q + kk + e;
+                        d[b][4 * q + e] = k >= k0 && k < k1 ? d[b][4 * q + e] : T(0);
+                    }
+            }
+        }
+        panel_mul<T, CBW, 2>(d, xb + r0, LDB, acc);
+        if (np > 0) {
+            int i = 0;
+            for (; i + PD <= np; i += PD) {
+#pragma unroll
+                for (int v = 0; v < PD; ++v) {
+                    const int nx = i + v + PD - 1;
+                    rows.load(ka + 32 * (nx < np ? nx : np - 1), f[(v + PD - 1) % PD]);
+                    panel_mul<T, CBW, 2>(f[v], xb + ka + 32 * (i + v), LDB, acc);
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < PD - 1; ++v)
+                if (i + v < np) panel_mul<T, CBW, 2>(f[v], xb + ka + 32 * (i + v), LDB, acc);
+        }
+        if (ka + 32 * np < kb && np >= 0 && ka < kb) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                panel_masked<T>(Mp, mrs, mcs, r0 + PR::row(b, lo), ka + 32 * np, 0, nbig, lane, d[b]);
+            panel_mul<T, CBW, 2>(d, xb + ka + 32 * np, LDB, acc);
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int r = r0 + PR::row(b, lo);
+#pragma unroll
+            for (int cb = 0; cb < CBW; ++cb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int c = cb * 16 + MF::di(lane, e);
+                    if (r < nbig && c < ncol) {
+                        const T v = unit ? acc.at(b, cb, e) + bs[c * LDB + r] : acc.at(b, cb, e);
+                        B[r * brs + c * bcs] = v * scale;
+                    }
+                }
+        }
+    }
+}
+
+template <typename T, int NBIG, int W, bool TRMM, bool KC>
+__global__ __launch_bounds__(PU_WAVES * 64) void panel_kernel(int nbig, int64_t m, const T *__restrict__ Mp,
+                                                              int64_t mrs, int64_t mcs, int lower, int unit,
+                                                              T *__restrict__ Bp, int64_t brs, int64_t bcs,
+                                                              const T *__restrict__ Wp, int64_t wrs, int64_t wcs,
+                                                              T scale, const int *__restrict__ Fp, unsigned *xmax) {
+    constexpr int LDB = NBIG + panel_pad<T>(), LDX = 64 + panel_pad<T>();
+    __shared__ __attribute__((aligned(16))) T strip[W * LDB];
+    const int64_t c0 = (int64_t)blockIdx.x * W;
+    if constexpr (TRMM) {
+        panel_trmm<T, NBIG, W, KC>(nbig, m, c0, Mp, mrs, mcs, lower != 0, unit != 0, Bp, brs, bcs, scale,
+                                   (NLA_LDS T *)strip);
+    } else {
+        __shared__ __attribute__((aligned(16))) T block[W * LDX];
+        const int64_t ncol = m - c0 < W ? m - c0 : W;
+        const int t = threadIdx.x;
+        PanelSolve<T, W, LDB, KC> P;
+        P.nbig = nbig;
+        P.nsb = (nbig + 63) / 64;
+        P.lane = t & 63;
+        P.wv = __builtin_amdgcn_readfirstlane(t >> 6);
+        P.lo = P.lane & 15;
+        P.kk = 4 * (P.lane >> 4);
+        P.lower = lower != 0;
+        P.unit = unit != 0;
+        P.Mp = Mp;
+        P.mrs = mrs;
+        P.mcs = mcs;
+        P.Wp = Wp;
+        P.wrs = wrs;
+        P.wcs = wcs;
+        P.Fp = Fp;
+        P.bs = (NLA_LDS T *)strip;
+        P.tmp = (NLA_LDS T *)block;
+        T *B = Bp + c0 * bcs;
+        panel_load<T, W, LDB>(B, brs, bcs, nbig, 64 * P.nsb, ncol, scale, P.bs);
+        __syncthreads();
+        if (P.wv < 4) P.template run<true>();
+        else P.template run<false>();
+        const T vmax = panel_store<T, W, LDB>(B, brs, bcs, nbig, ncol, P.bs);
+        if constexpr (sizeof(T) == 4) {
+            if (xmax != nullptr) {
+                // one global atomic per work-group: every work-group of the
+                // launch targets the same slot, and one per wave serialized
+                // there (+10 us per launch)
+                __shared__ unsigned s_max;
+                unsigned b = __float_as_uint((float)vmax);
+                for (int o = 32; o > 0; o >>= 1) {
+                    const unsigned u = __shfl_xor(b, o);
+                    b = u > b ? u : b;
+                }
+                if (t == 0) s_max = 0u;
+                __syncthreads();
+                if ((t & 63) == 0) atomicMax(&s_max, b);
+                __syncthreads();
+                if (t == 0 && s_max != 0u) atomicMax(xmax, s_max);
+            }
+        }
+    }
+}
+
+template <typename T, int NBIG, int W, bool KC>
+static hipError_t launch_panel_k(const PanelArgs<T> &a, hipStream_t s) {
+    const dim3 grid((unsigned)((a.m + W - 1) / W)), block(PU_WAVES * 64);
     const int lo = a.lower ? 1 : 0, un = a.unit ? 1 : 0;
     if (a.trmm)
-        hipLaunchKernelGGL((panel_kernel<T, NBIG, W, true, NW>), dim3((unsigned)groups), dim3(NW * 64), 0, s,
-                           a.nbig, a.m, a.M, a.mrs, a.mcs, lo, un, a.B, a.brs, a.bcs, a.W, a.wrs, a.wcs, a.scale,
-                           (const int *)nullptr, (unsigned *)nullptr);
+        hipLaunchKernelGGL((panel_kernel<T, NBIG, W, true, KC>), grid, block, 0, s, a.nbig, a.m, a.M, a.mrs, a.mcs,
+                           lo, un, a.B, a.brs, a.bcs, a.W, a.wrs, a.wcs, a.scale, (const int *)nullptr,
+                           (unsigned *)nullptr);
     else
-        hipLaunchKernelGGL((panel_kernel<T, NBIG, W, false, NW>), dim3((unsigned)groups), dim3(NW * 64), 0, s,
-                           a.nbig, a.m, a.M, a.mrs, a.mcs, lo, un, a.B, a.brs, a.bcs, a.W, a.wrs, a.wcs, a.scale,
-                           a.F, a.xmax);
+        hipLaunchKernelGGL((panel_kernel<T, NBIG, W, false, KC>), grid, block, 0, s, a.nbig, a.m, a.M, a.mrs, a.mcs,
+                           lo, un, a.B, a.brs, a.bcs, a.W, a.wrs, a.wcs, a.scale, a.F, a.xmax);
     return hipGetLastError();
 }
 
-// Panels up to 512 rows use the 512-row LDS strip (4 or 8 waves); larger
-// ones (up to PANEL_MAX) the 1024-row strip with 4 waves, whose FP64 form
-// only fits LDS with 16 columns per work-group.
+// The strip's LDS is sized for 128, 256 or 512 rows.
+template <typename T, int W>
+static hipError_t launch_panel_w(const PanelArgs<T> &a, hipStream_t s) {
+    const bool kc = a.mcs == 1;
+    if (a.nbig <= 128) return kc ? launch_panel_k<T, 128, W, true>(a, s) : launch_panel_k<T, 128, W, false>(a, s);
+    if (a.nbig <= 256) return kc ? launch_panel_k<T, 256, W, true>(a, s) : launch_panel_k<T, 256, W, false>(a, s);
+    return kc ? launch_panel_k<T, 512, W, true>(a, s) : launch_panel_k<T, 512, W, false>(a, s);
+}
+
+template <typename T, int NBIG, bool TRMM>
+static hipError_t launch_panel_left(const PanelArgs<T> &a, hipStream_t s) {
+    hipLaunchKernelGGL((panel_left_kernel<T, NBIG, 16, TRMM>), dim3((unsigned)((a.m + 15) / 16)), dim3(256), 0, s,
+                       a.nbig, a.m, a.M, a.mrs, a.mcs, a.lower ? 1 : 0, a.unit ? 1 : 0, a.B, a.brs, a.bcs, a.W, a.wrs,
+                       a.wcs, a.scale, TRMM ? nullptr : a.F, TRMM ? nullptr : a.xmax);
+    return hipGetLastError();
+}
+
+template <typename T, bool TRMM>
+static hipError_t launch_panel_left_n(const PanelArgs<T> &a, hipStream_t s) {
+    if (a.nbig <= 128) return launch_panel_left<T, 128, TRMM>(a, s);
+    if (a.nbig <= 256) return launch_panel_left<T, 256, TRMM>(a, s);
+    if (a.nbig <= 512) return launch_panel_left<T, 512, TRMM>(a, s);
+    return launch_panel_left<T, 1024, TRMM>(a, s);
+}
+
 template <typename T>
 hipError_t launch_panel(const PanelArgs<T> &a, hipStream_t s) {
     if (a.m <= 0 || a.nbig <= 0) return hipSuccess;
     if (a.nbig > PANEL_MAX) return hipErrorInvalidValue;
     if (a.strip != 16 && a.strip != 32) return hipErrorInvalidValue;
-    if (a.waves != 4 && a.waves != 8) return hipErrorInvalidValue;
-    if (a.nbig <= 512) {
-        if (a.waves == 8)
-            return a.strip == 32 ? launch_panel_w<T, 512, 32, 8>(a, s) : launch_panel_w<T, 512, 16, 8>(a, s);
-        return a.strip == 32 ? launch_panel_w<T, 512, 32, 4>(a, s) : launch_panel_w<T, 512, 16, 4>(a, s);
-    }
-    if constexpr (sizeof(T) == 4) {
-        if (a.strip == 32) return launch_panel_w<T, 1024, 32, 4>(a, s);
-    }
-    return launch_panel_w<T, 1024, 16, 4>(a, s);
+    // Four waves and 16 columns leave room for two and more work-groups on a
+    // CU: the left-looking strip wins where there are more strips than CUs, or
+    // no chain to shorten.  Measured on MI355X (us, left / eight waves): FP64
+    // TRSM of 512 rows with 64 / 4096 / 8192 columns 40.2 / 32.8, 47.9 / 41.0,
+    // 75.0 / 80.8, 128 rows 7.0 / 7.5, 64 rows 4.4 / 4.5; FP64 TRMM 512 rows
+    // 37.8 / 23.8, 45.5 / 30.8, 72.6 / 59.8, 128 rows 6.7 / 5.8 and with 8192
+    // columns 11.2 / 12.2; FP32 TRSM 512 rows 27.6 / 22.9, 30.9 / 26.1,
+    // 46.6 / 49.7, TRMM 27.1 / 17.9, 30.1 / 22.3, 47.7 / 43.8.
+    const bool many = a.m > 16 * 256, small = a.nbig <= 128;
+    if (a.nbig > PU_MAX || a.waves == 4 || (a.waves == 0 && (a.trmm ? many && small : many || small)))
+        return a.trmm ? launch_panel_left_n<T, true>(a, s) : launch_panel_left_n<T, false>(a, s);
+    return a.strip == 32 ? launch_panel_w<T, 32>(a, s) : launch_panel_w<T, 16>(a, s);
 }
 
 template hipError_t launch_panel<float>(const PanelArgs<float> &, hipStream_t);

@@ -341,3 +341,43 @@ def test_full_size_8192(nla, dt):
         assert rel < 1e3 * eps(npdt), rel
         del A, B, B0
         torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [2, 31, 33, 65, 129, 159, 161, 193, 257, 320, 449, 511, 512])
+def test_eight_wave_panels(nla, dt, n):
+    """The eight-wave panels at the edges of their 32-row units and 64-row
+    blocks, every side / uplo / trans, TRSM and TRMM, unit and general
+    diagonals, column counts around a strip: the oracle's bounds.  The other
+    triangle (and a unit diagonal) holds NaN, which must not be used, and a
+    column of B holds an infinity, which must stay in that column's result."""
+    from nextla_amd import _lib
+    old_w = _lib.set_config(_lib.NLA_CFG_PANEL_WAVES, 8)
+    rows_key = _lib.NLA_CFG_PANEL_ROWS_F64 if dt == np.float64 else _lib.NLA_CFG_PANEL_ROWS_F32
+    old_r = _lib.set_config(rows_key, 512)
+    try:
+        rng = np.random.default_rng(n)
+        for (side, uplo, trans, func), diag, m in itertools.product(itertools.product("LR", "LU", "NT", "SM"), "NU",
+                                                                   (15, 17)):
+            T = np.tril(rng.uniform(-1, 1, (n, n)) / np.sqrt(n), -1)
+            np.fill_diagonal(T, 1.0 if diag == "U" else 2 + rng.random(n))
+            A = np.asfortranarray((T if uplo == "L" else T.T).astype(dt))
+            B = rng.standard_normal((n, m) if side == "L" else (m, n)).astype(dt)
+            P = np.array(A)
+            P[np.triu_indices(n, 1) if uplo == "L" else np.tril_indices(n, -1)] = np.nan
+            if diag == "U":
+                np.fill_diagonal(P, np.nan)
+            Binf = np.array(B)
+            Binf[(n - 1, m - 1) if side == "L" else (m - 1, n - 1)] = np.inf
+            res = []
+            for rhs in (B, Binf):
+                Ad, Bd = (torch.from_numpy(np.ascontiguousarray(t.T)).cuda().t() for t in (P, rhs))
+                (nla.trsm if func == "S" else nla.trmm)(side, uplo, trans, diag, Ad, Bd, 1.5)
+                res.append(Bd.cpu().numpy())
+            check_bound(side, uplo, trans, 1.5, func, A, B, res[0])
+            keep = (slice(None), slice(0, m - 1)) if side == "L" else (slice(0, m - 1), slice(None))
+            assert np.array_equal(res[0][keep], res[1][keep])
+            assert not np.all(np.isfinite(res[1]))
+    finally:
+        _lib.set_config(_lib.NLA_CFG_PANEL_WAVES, old_w)
+        _lib.set_config(rows_key, old_r)
