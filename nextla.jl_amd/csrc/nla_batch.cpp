@@ -96,7 +96,6 @@ static Layout layout_of(char func, int32_t dtype, const nla_batch_item *items, i
 // cls 5: the FP64 GEMMs of few right-hand sides, in narrow tiles).
 struct Launch {
     int stage, cls, start, count, groups;
-    bool vec;
 };
 
 }  // namespace nla
@@ -117,7 +116,6 @@ struct nla_batch_plan_s {
 
 namespace nla {
 
-static inline bool al16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 // The host side of a plan: descriptors, tasks and the launch partition
 // (grid sizes come later, from the device's occupancy).  Besides what the
@@ -343,19 +341,14 @@ static int32_t plan_host(char side, char uplo, char trans, char func, const nla_
             while (pt < ptasks.size() && pan_stage[(size_t)ptasks[pt].sys] == s &&
                    cls_of(pan[(size_t)ptasks[pt].sys].n) == c)
                 ++pt;
-            if (pt > start) H.launches.push_back(Launch{s, c, (int)start, (int)(pt - start), 0, false});
+            if (pt > start) H.launches.push_back(Launch{s, c, (int)start, (int)(pt - start), 0});
         }
         for (int nw = 0; nw < 2; ++nw) {  // wide tiles (cls 4), then narrow ones (cls 5)
             const size_t start = gt;
-            bool vec = true;
             while (gt < gtasks.size() && gem_stage[(size_t)gtasks[gt].x] == s &&
-                   H.gem_narrow[(size_t)gtasks[gt].x] == nw) {
-                const GroupGemm<T> &g = gem[(size_t)gtasks[gt].x];
-                constexpr int V = 16 / sizeof(T);
-                vec = vec && al16(g.X) && al16(g.Y) && g.ldx % V == 0 && g.ldy % V == 0;
+                   H.gem_narrow[(size_t)gtasks[gt].x] == nw)
                 ++gt;
-            }
-            if (gt > start) H.launches.push_back(Launch{s, 4 + nw, (int)start, (int)(gt - start), 0, vec});
+            if (gt > start) H.launches.push_back(Launch{s, 4 + nw, (int)start, (int)(gt - start), 0});
         }
     }
     // a perturbed task order within every launch (testing: a task's result
@@ -399,7 +392,7 @@ static int32_t build(char side, char uplo, char trans, char func, const nla_batc
     P->launches = H.launches;
     for (Launch &l : P->launches)
         l.groups = l.cls < 4 ? grid(batch_kernel_ptr<T>(trmm, BATCH_CLASSES[l.cls]), l.count)
-                             : grid(grouped_gemm_ptr<T>(P->tx, P->ty, l.vec, P->rows_m, l.cls == 5), l.count);
+                             : grid(grouped_gemm_ptr<T>(P->tx, P->ty, P->rows_m, l.cls == 5), l.count);
     // one staged image of the descriptor region, copied in stream order
     P->host.assign((size_t)(L.inv - L.sys), 0);
     char *h = P->host.data() - L.sys;
@@ -433,7 +426,7 @@ static hipError_t enqueue(nla_batch_plan_s *P, hipStream_t s) {
         if (l.cls < 4)
             e = launch_batch<T>(pan, ptasks + l.start, l.count, ctr, P->trmm, BATCH_CLASSES[l.cls], l.groups, s);
         else
-            e = launch_grouped_gemm<T>(gem, gtasks + l.start, l.count, ctr, P->tx, P->ty, l.vec, P->rows_m,
+            e = launch_grouped_gemm<T>(gem, gtasks + l.start, l.count, ctr, P->tx, P->ty, P->rows_m,
                                        l.cls == 5, l.groups, s);
     }
     return e;

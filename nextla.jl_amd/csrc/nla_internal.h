@@ -131,13 +131,12 @@ inline int group_tile_n(bool rows_m, int elem_bytes, bool narrow) {
 }
 
 // Persistent grouped GEMM over tasks (gemm index, tile index) taken from a
-// counter (cleared by a kernel first); vec: every X and Y of the launch has
-// 16-byte aligned columns and leading dimensions.
+// counter (cleared by a kernel first).
 template <typename T>
 hipError_t launch_grouped_gemm(const GroupGemm<T> *g, const int2 *tasks, int ntasks, int *counter, bool tx, bool ty,
-                               bool vec, bool rows_m, bool narrow, int groups, hipStream_t s);
+                               bool rows_m, bool narrow, int groups, hipStream_t s);
 template <typename T>
-const void *grouped_gemm_ptr(bool tx, bool ty, bool vec, bool rows_m, bool narrow);
+const void *grouped_gemm_ptr(bool tx, bool ty, bool rows_m, bool narrow);
 
 // One system of a batch in the panel's canonical form (see PanelArgs).
 template <typename T>
