@@ -24,11 +24,11 @@ namespace nla {
 #define NLA_LDS __attribute__((address_space(3)))
 
 // EDGE: the tile may reach past the operand's last outer index (no).  What
-// lies past it only feeds results that are not stored, so addresses are
-// clamped and nothing is zeroed; a chunk that straddles the end is read from
-// no - VW on and shifted into place at the LDS store.  k is in range in
-// load(); load_tail() takes the last, partial step and zeroes what is past K
-// (in both operands: no 0 * NaN).
+// lies past it only feeds results that are not stored, so load() clamps whole
+// chunks into the operand, zeroes nothing, and lets a chunk that straddles
+// the end run on into the next k (memory of the operand while VW and more k
+// remain: the caller takes the last steps with load_tail()).  load_tail()
+// checks every element and zeroes what is past K, in both operands: no 0 * NaN.
 template <typename T, int BO, int BK, int NT, bool KCONTIG, bool EDGE>
 struct TileLoader {
     // Each thread moves CH chunks of VW consecutive elements along the
@@ -44,10 +44,9 @@ struct TileLoader {
     typedef T lvec_t __attribute__((ext_vector_type(VW)));
 
     T r[CH][VW];
-    const T *p[CH];  // the chunks' addresses at the next step
-    int shift[EDGE && !KCONTIG ? CH : 1];
+    const T *p[CH];  // the chunks' addresses at the first step
+    int last[EDGE && !KCONTIG ? CH : 1];  // the chunk's last element inside the operand
     int64_t ks;
-    int narrow;        // outer indices when fewer than VW (no whole chunk to read), else 0
     uint32_t okbits;   // load_tail: bit (c*VW+e) set when the element's k is in range
 
     // Coordinates (outer, k) inside the tile of chunk c of thread t.
@@ -67,7 +66,6 @@ struct TileLoader {
     __device__ inline void init(const T *__restrict__ P, int64_t so, int64_t sk, int64_t o0, int64_t k0, int64_t no,
                                 int t) {
         ks = sk;
-        narrow = EDGE && !KCONTIG && no < VW ? (int)no : 0;
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             int o, k;
@@ -75,30 +73,26 @@ struct TileLoader {
             int64_t go = o0 + o;
             if constexpr (EDGE && KCONTIG) go = go < no ? go : no - 1;
             if constexpr (EDGE && !KCONTIG) {
-                const int64_t last = no > VW ? no - VW : 0, s = go < last ? go : last;
-                shift[c] = go - s < VW ? (int)(go - s) : VW - 1;
-                go = s;
+                if (go >= no) go = no - 1;
+                last[c] = no - 1 - go < VW - 1 ? (int)(no - 1 - go) : VW - 1;
             }
             p[c] = P + go * so + (k0 + k) * sk;
         }
     }
-    __device__ inline void load() {
+    // Step kt (uniform: its offset is added in scalar registers).
+    __device__ inline void load(int kt) {
+        const int64_t off = (int64_t)kt * BK * ks;
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
-            if (EDGE && !KCONTIG && narrow) {
+            const gvec_t v = *reinterpret_cast<const gvec_t *>(p[c] + off);
 #pragma unroll
-                for (int e = 0; e < VW; ++e) r[c][e] = p[c][e < narrow ? e : 0];
-            } else {
-                const gvec_t v = *reinterpret_cast<const gvec_t *>(p[c]);
-#pragma unroll
-                for (int e = 0; e < VW; ++e) r[c][e] = v[e];
-            }
-            p[c] += (int64_t)BK * ks;
+            for (int e = 0; e < VW; ++e) r[c][e] = v[e];
         }
     }
-    // The last step, of which nk (1 .. BK - 1) k remain; an element past them
-    // reads its row's first k of the step.
-    __device__ inline void load_tail(int nk, int t) {
+    // Step kt, of which nk (1 .. BK) k remain; an element past them reads its
+    // outer index's first k of the step.
+    __device__ inline void load_tail(int kt, int nk, int t) {
+        const int64_t off = (int64_t)kt * BK * ks;
         okbits = 0;
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
@@ -107,8 +101,9 @@ struct TileLoader {
 #pragma unroll
             for (int e = 0; e < VW; ++e) {
                 const bool ok = (KCONTIG ? k + e : k) < nk;
-                if constexpr (KCONTIG) r[c][e] = p[c][ok ? e : -k];
-                else r[c][e] = (ok ? p[c] : p[c] - (int64_t)k * ks)[EDGE && narrow && e >= narrow ? 0 : e];
+                const T *q = p[c] + off;
+                if constexpr (KCONTIG) r[c][e] = q[ok ? e : -k];
+                else r[c][e] = (ok ? q : q - (int64_t)k * ks)[EDGE && e > last[c] ? last[c] : e];
                 okbits |= (ok ? 1u : 0u) << (c * VW + e);
             }
         }
@@ -120,20 +115,6 @@ struct TileLoader {
 #pragma unroll
             for (int e = 0; e < VW; ++e)
                 if (!((okbits >> (c * VW + e)) & 1u)) r[c][e] = T(0);
-    }
-
-    // A straddling chunk was read from no - VW on: element e sits shift later.
-    __device__ inline void align() {
-        if constexpr (EDGE && !KCONTIG) {
-#pragma unroll
-            for (int c = 0; c < CH; ++c)
-#pragma unroll
-                for (int s = 1; s < VW; s <<= 1)
-                    if (shift[c] & s) {
-#pragma unroll
-                        for (int e = 0; e + s < VW; ++e) r[c][e] = r[c][e + s];
-                    }
-        }
     }
 
     // Zero the elements outside a triangle: keep (outer, k) when
@@ -238,8 +219,8 @@ __device__ __forceinline__ void gemm_tile(int64_t M, int64_t N, int64_t K, T alp
     if (TRI == 3) kbeg = col0 < K ? col0 : K;
     if (TRI == 4) kend = col0 + BN < K ? col0 + BN : K;
     if (TRI == 5) kbeg = row0 > col0 ? row0 : col0;
-    const int nfull = (int)((kend - kbeg) / BK), tail = (int)((kend - kbeg) % BK);
-    const int nkt = nfull + (tail ? 1 : 0);
+    const int64_t kn = kend - kbeg, whole = EDGE ? kn - LX::VW : kn;
+    const int nfull = whole > 0 ? (int)(whole / BK) : 0, nkt = (int)((kn + BK - 1) / BK);
 
     LX lx;
     LY ly;
@@ -247,46 +228,23 @@ __device__ __forceinline__ void gemm_tile(int64_t M, int64_t N, int64_t K, T alp
     // Y[c + k*ldy] : Y[k + c*ldy]
     lx.init(X, TX ? ldx : 1, TX ? 1 : ldx, row0, kbeg, M, t);
     ly.init(Y, TY ? 1 : ldy, TY ? ldy : 1, col0, kbeg, N, t);
-    auto fetch = [&](int kt) {
-        if (kt < nfull) {
-            lx.load();
-            ly.load();
-        } else {
-            lx.load_tail(tail, t);
-            ly.load_tail(tail, t);
-        }
-    };
     // op(X)(r,k): outer r, inner k.  op(Y)(k,c): outer c, inner k; the Y
     // triangle conditions are c <= k (lower) / c >= k (upper).  Only steps
     // that meet the diagonal need a mask.
     auto stage = [&](int kt, int buf) {
         const int64_t k0 = kbeg + (int64_t)kt * BK;
-        if (kt >= nfull) {
-            lx.apply_bounds();
-            ly.apply_bounds();
-        }
-        lx.align();
-        ly.align();
         if (TRI == 1 && k0 + BK > row0) lx.template mask<true>(row0, k0, t);
         if ((TRI == 2 || TRI == 5) && k0 < row0 + BM) lx.template mask<false>(row0, k0, t);
         if ((TRI == 3 || TRI == 5) && k0 < col0 + BN) ly.template mask<false>(col0, k0, t);
         if (TRI == 4 && k0 + BK > col0) ly.template mask<true>(col0, k0, t);
         lx.store(lds_x[buf], t);
+        __builtin_amdgcn_sched_barrier(0);  // the stores in the order of the loads: each waits for its own
         ly.store(lds_y[buf], t);
     };
-    if (nkt > 0) {
-        fetch(0);
-        stage(0, 0);
-    }
-    __syncthreads();
-
     const int lo = lane % MF::BD, lk = lane / MF::BD;
-    for (int kt = 0; kt < nkt; ++kt) {
-        const int cur = kt & 1;
-        const bool more = kt + 1 < nkt;
-        if (more) fetch(kt + 1);
-        const NLA_LDS T *sx = lds_x[cur];
-        const NLA_LDS T *sy = lds_y[cur];
+    auto multiply = [&](int buf) {
+        const NLA_LDS T *sx = lds_x[buf];
+        const NLA_LDS T *sy = lds_y[buf];
         __builtin_amdgcn_s_setprio(1);  // issue priority to waves in their MFMA cluster
 #pragma unroll
         for (int ks = 0; ks < BK; ks += MF::KD) {
@@ -301,7 +259,36 @@ __device__ __forceinline__ void gemm_tile(int64_t M, int64_t N, int64_t K, T alp
                 for (int rb = 0; rb < RB; ++rb) acc[cb][rb] = MF::mma(a[cb], b[rb], acc[cb][rb]);
         }
         __builtin_amdgcn_s_setprio(0);
+    };
+    // whole steps, the next one's loads in flight behind the products
+    if (nfull > 0) {
+        lx.load(0);
+        ly.load(0);
+        stage(0, 0);
+    }
+    __syncthreads();
+    for (int kt = 0; kt < nfull; ++kt) {
+        const int cur = kt & 1;
+        const bool more = kt + 1 < nfull;
+        if (more) {
+            lx.load(kt + 1);
+            ly.load(kt + 1);
+        }
+        multiply(cur);
         if (more) stage(kt + 1, cur ^ 1);
+        __syncthreads();
+    }
+    // the checked ones (at most two), on their own: a choice of loads inside
+    // the loop above made the compiler wait for them before the products
+    for (int kt = nfull; kt < nkt; ++kt) {
+        const int64_t left = kn - (int64_t)kt * BK;
+        lx.load_tail(kt, left < BK ? (int)left : BK, t);
+        ly.load_tail(kt, left < BK ? (int)left : BK, t);
+        lx.apply_bounds();
+        ly.apply_bounds();
+        stage(kt, kt & 1);
+        __syncthreads();
+        multiply(kt & 1);
         __syncthreads();
     }
 
