@@ -64,3 +64,28 @@ def test_large_self_certified(nla):
     got = torch.tril(A)
     assert (torch.linalg.norm(got - ref) / torch.linalg.norm(ref)).item() <= 1e-14
     assert torch.equal(torch.triu(A, 1), torch.triu(A0, 1))
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [129, 159, 161, 255, 257, 511, 1025, 3071, 3072, 3137])
+def test_tile_edges_and_other_triangle(nla, dtype, n):
+    """Sizes at the edges of the 32- and 64-wide tiles and of the rule between
+    them, lda > n: the triangle within (n + 2) eps sum |L||L| of the product in
+    float64 (any order of the sums), NaN in the other triangle not used and
+    left as it is."""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(n)
+    for uplo in "LU":
+        big = torch.empty((n, n + 5), dtype=dtype, device=DEV).normal_(generator=g).t()
+        A = big[:n]
+        tri = torch.tril(A.double()) if uplo == "L" else torch.triu(A.double())
+        A.masked_fill_(torch.triu(torch.ones(n, n, dtype=torch.bool, device=DEV), 1) if uplo == "L"
+                       else torch.tril(torch.ones(n, n, dtype=torch.bool, device=DEV), -1), float("nan"))
+        keep, pad = A.clone(), big[n:].clone()
+        nla.lauum_(uplo, n, A)
+        a, b = (tri.t(), tri) if uplo == "L" else (tri, tri.t())
+        ref, bound = a @ b, (n + 2) * torch.finfo(dtype).eps * (a.abs() @ b.abs())
+        mask = torch.isnan(keep)
+        assert torch.all(torch.isnan(A) == mask)
+        assert torch.all(((A.double() - ref).abs() <= bound) | mask)
+        assert torch.equal(big[n:], pad)
