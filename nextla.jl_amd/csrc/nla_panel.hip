@@ -764,16 +764,18 @@ struct PanelSolve {
             for (int e = 0; e < 4; ++e)
                 bs[(cb * 16 + MF::di(lane, e)) * LDB + r0] = r0 < nbig ? x.at(0, cb, e) : T(0);
     }
-    // An ill-conditioned diagonal block: X += inv(M_ss) (B_s - M_ss X).  A
-    // rare path; every wave passes its barriers.
+    // An ill-conditioned diagonal block: X += inv(M_ss) (B_s - M_ss X).  The
+    // correction has sums of its own: the two sets that hold X may be far
+    // larger than X, and would round what is added to them at their size.
+    // Every wave passes the barriers.
     template <bool DIAG>
     __device__ inline void refine(int s, X &x) {
         const int bl = block(s), nb = bl == nsb - 1 ? nbig - 64 * bl : 64, i = 16 * wv + lo, r = 64 * bl + i;
-        X v;
-        T res[CBW][4];
+        T x0[CBW][4];
         if (DIAG) put_x(s, x);
-        __syncthreads();
+        __syncthreads();  // X complete, and every wave's product with B_s done
         if (DIAG) {
+            X v;
             v.zero();
             const int ka = lower ? 0 : (unit ? i + 1 : i), kb = i < nb ? (lower ? (unit ? i : i + 1) : nb) : 0;
 #pragma unroll
@@ -787,21 +789,21 @@ struct PanelSolve {
             for (int cb = 0; cb < CBW; ++cb)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int c = cb * 16 + MF::di(lane, e);
-                    const T mx = unit && i < nb ? v.at(0, cb, e) + x.at(0, cb, e) : v.at(0, cb, e);
-                    res[cb][e] = tmp[c * LDX + i] - mx;
+                    NLA_LDS T *p = tmp + (cb * 16 + MF::di(lane, e)) * LDX + i;  // this lane's own element of B_s
+                    x0[cb][e] = x.at(0, cb, e);
+                    const T mx = unit ? v.at(0, cb, e) + x0[cb][e] : v.at(0, cb, e);
+                    *p = i < nb ? *p - mx : T(0);
                 }
         }
         __syncthreads();
         if (DIAG) {
+            x.zero();
+            apply_inverse(x);
 #pragma unroll
             for (int cb = 0; cb < CBW; ++cb)
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    tmp[(cb * 16 + MF::di(lane, e)) * LDX + i] = i < nb ? res[cb][e] : T(0);
+                for (int e = 0; e < 4; ++e) x.a[0][0][cb][e] = x0[cb][e] + x.at(0, cb, e), x.a[1][0][cb][e] = T(0);
         }
-        __syncthreads();
-        if (DIAG) apply_inverse(x);
     }
     // Solves block s into the strip: sums out, inverse, X in; two barriers.
     template <bool DIAG>
