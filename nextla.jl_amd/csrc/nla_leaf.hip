@@ -142,23 +142,48 @@ __global__ __launch_bounds__(LEAF_COLS) void leaf_kernel(int nb, int64_t m, cons
     }
 }
 
+// 16 x 16 x 4 MFMA: step s of a lane in group kk = lane / 16 takes k =
+// kmap(kk, s), which is also the row of its result register s.
+template <typename T>
+struct Mma16;
+template <>
+struct Mma16<double> {
+    typedef d4_t acc_t;
+    __device__ static inline acc_t mma(double a, double b, acc_t c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    __device__ static inline int kmap(int kk, int s) { return 4 * s + kk; }
+    static constexpr double big = 0x1p500;
+};
+template <>
+struct Mma16<float> {
+    typedef f4_t acc_t;
+    __device__ static inline acc_t mma(float a, float b, acc_t c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    __device__ static inline int kmap(int kk, int s) { return 4 * kk + s; }
+    static constexpr float big = 0x1p60f;
+};
+
 // Inverse of one 64 x 64 triangular block with 256 threads, in three stages
 // (the blocked scheme of LAPACK's trtri), in place in LDS:
 //   1. the four 16 x 16 diagonal sub-blocks by substitution on the columns of
-//      the identity (64 lanes, one column each, 16-step chains), written over
-//      the sub-blocks once every lane has read them;
+//      the identity (64 lanes, one column each, 16-step chains);
 //   2. 32 x 32 inverses: inv([A 0; C B]) = [inv A, 0; -inv B * C * inv A, inv B],
-//      C * inv A through the scratch st, the result written over C;
+//      on MFMA, the result written over C;
 //   3. the same step from 32 to 64.
-// sl: the canonical lower block (column-major, 64 x 64), which becomes its
-// inverse; st: 32 x 32 scratch.  The parts above the diagonal stay zero, so
-// the products run over full, unrolled k ranges and the extra terms add
-// exact zeros.  Upper blocks are inverted as J U J.  40 KB of LDS in FP64
-// (four work-groups per CU; with a separate inverse it was 72 KB, two).
+// sl: the canonical lower block (column-major, leading dimension TRTRI_LD),
+// which becomes its inverse; sp: TRTRI_SP scratch.  The parts above the
+// diagonal stay zero, so the products run over full k ranges and the extra
+// terms add exact zeros.  Upper blocks are inverted as J U J.  A call of one
+// block is bound by its chain (loads, 16 quotients, two product stages), the
+// batched form by LDS traffic: with the products in FMAs a thread read two
+// LDS words per multiply.  38 KB of LDS in FP64, four work-groups per CU.
+constexpr int TRTRI_LD = 66, TRTRI_SP = 576;
 template <typename T>
 __device__ __forceinline__ void trtri64_block(int64_t n, int64_t blk, const T *__restrict__ A, int64_t rs, int64_t cs, bool lower,
-                              bool unit, T *__restrict__ W, T *sl, T *st, int *__restrict__ F) {
-    constexpr int NB = 64, NT = 256;
+                              bool unit, T *__restrict__ W, T *sl, T *sp, int *__restrict__ F) {
+    constexpr int NB = 64, NT = 256, LD = TRTRI_LD;
     const int t = threadIdx.x;
     const int64_t off = blk * NB;
     const int nb = (int)(n - off < NB ? n - off : NB);
@@ -184,129 +209,145 @@ __device__ __forceinline__ void trtri64_block(int64_t n, int64_t blk, const T *_
         const int e = t + u * NT;
         const int i = arow ? e % NB : e / NB;
         const int j = arow ? e / NB : e % NB;
-        sl[j * NB + i] = v[u];
+        sl[j * LD + i] = v[u];
     }
     __syncthreads();
-    // ||L||_1 (largest column sum) while L is still there: wave 0, lane = column
-    // (lane t walks its column from row t on, so that the 64 lanes of a read
-    // fall in different banks rather than all in one)
-    T nl = T(0);
-    if (F != nullptr && t < NB) {
-#pragma unroll 8
-        for (int i = 0; i < NB; ++i) {
-            const T a = sl[t * NB + ((i + t) & (NB - 1))];
-            nl += a < T(0) ? -a : a;
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            const T other = __shfl_xor(nl, o);
-            nl = other > nl ? other : nl;
-        }
-    }
-    // 1. sub-block b, column c: y = inv(D_b) e_c
-    T x[16];
-    const int b1 = t >> 4, c1 = t & 15, o1 = 16 * b1;
+    // Column sums of |L| for ||L||_1: thread t adds 16 rows of column t % 64
+    // (walked from a lane-dependent row, so that the lanes of a read fall in
+    // different banks).  sp: partial sums of L, of inv(L), reciprocals.
+    const int lane = t & 63, wv = t >> 6;
+    auto partial_sums = [&](T *part) {
+        T a = T(0);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) a += fabs(sl[lane * LD + 16 * wv + ((u + lane) & 15)]);
+        part[t] = a;
+    };
+    T *rinv = sp + 512;
+    if (F != nullptr) partial_sums(sp);
+    // 1. inverses of the 16 x 16 diagonal blocks b: lane (b, c) solves D_b y =
+    // e_c.  Each of its 16 quotients is a product with the reciprocal of the
+    // diagonal and one correction by the exact remainder (the quotient
+    // rounded, as a division gives it, in three dependent operations instead
+    // of a division's dozen); a block with an entry whose reciprocal or
+    // remainder could leave the normal range takes the divisions.
     if (t < 64) {
+        const T d = sl[t * LD + t], ad = fabs(d);
+        constexpr T big = Mma16<T>::big, small = T(1) / big;
+        const bool plain = __all(ad >= small && ad <= big);
+        rinv[t] = T(1) / d;
+        T x[16];
+        const int o1 = 16 * (t >> 4), c1 = t & 15;
+        __builtin_amdgcn_wave_barrier();
+        T *blk16 = sl + o1 * LD + o1;
 #pragma unroll
         for (int i = 0; i < 16; ++i) x[i] = (i == c1) ? T(1) : T(0);
+        if (plain) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            x[j] = x[j] / sl[(o1 + j) * NB + o1 + j];
+            for (int j = 0; j < 16; ++j) {
+                const T dj = blk16[j * LD + j], rj = rinv[o1 + j];
+                const T q = x[j] * rj;
+                x[j] = fma(fma(-q, dj, x[j]), rj, q);
 #pragma unroll
-            for (int r = j + 1; r < 16; ++r) x[r] -= sl[(o1 + j) * NB + o1 + r] * x[j];
+                for (int r = j + 1; r < 16; ++r) x[r] -= blk16[j * LD + r] * x[j];
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                x[j] = x[j] / blk16[j * LD + j];
+#pragma unroll
+                for (int r = j + 1; r < 16; ++r) x[r] -= blk16[j * LD + r] * x[j];
+            }
         }
-    }
-    __syncthreads();  // every lane has read its sub-block
-    if (t < 64) {
+        __builtin_amdgcn_wave_barrier();  // one wave, in order: every lane has read its block
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sl[(o1 + c1) * NB + o1 + i] = x[i];
-    }
-    __syncthreads();
-    // 2. two 32-blocks p: st_p = C_p * inv(D_2p) (16 x 16), then
-    //    C_p <- -inv(D_2p+1) * st_p.  Thread t: block p = t>>7, row i,
-    //    columns j and j+8.
-    {
-        const int p = t >> 7, q = t & 127, i = q & 15, j = q >> 4, o = 32 * p;
-        T a0 = T(0), a1 = T(0);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const T c = sl[(o + k) * NB + o + 16 + i];
-            a0 += c * sl[(o + j) * NB + o + k];
-            a1 += c * sl[(o + j + 8) * NB + o + k];
-        }
-        st[p * 256 + j * 16 + i] = a0;
-        st[p * 256 + (j + 8) * 16 + i] = a1;
-        __syncthreads();  // C_p read by every lane; st_p complete
-        a0 = T(0);
-        a1 = T(0);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const T c = sl[(o + 16 + k) * NB + o + 16 + i];
-            a0 += c * st[p * 256 + j * 16 + k];
-            a1 += c * st[p * 256 + (j + 8) * 16 + k];
-        }
-        sl[(o + j) * NB + o + 16 + i] = -a0;
-        sl[(o + j + 8) * NB + o + 16 + i] = -a1;
+        for (int i = 0; i < 16; ++i) blk16[c1 * LD + i] = x[i];
     }
     __syncthreads();
-    // 3. st = Q * inv(P) (32 x 32, inv(P) lower), Q <- -inv(R) * st.
-    //    Thread t: row i = t & 31, columns j0 + 8u.
-    {
-        const int i = t & 31, j0 = t >> 5;
-        T a[4] = {T(0), T(0), T(0), T(0)};
+    // Products of 16 x 16 blocks on MFMA.  A result's registers are the right
+    // operand of the next product as they stand (step s of lane l takes k =
+    // kmap(l / 16, s)), so C inv(D) never goes through LDS.
+    typedef Mma16<T> MM;
+    typename MM::acc_t step3[2];
+    const int lo = lane & 15, kk = lane >> 4;
+    // acc += L(rows r0.., cols c0..) * x, or * L(rows c0.., cols d0..)
+    auto left = [&](int r0, int c0, const typename MM::acc_t &x, typename MM::acc_t acc) {
 #pragma unroll
-        for (int k = 0; k < 32; ++k) {
-            const T c = sl[k * NB + 32 + i];
+        for (int s = 0; s < 4; ++s) acc = MM::mma(sl[(c0 + MM::kmap(kk, s)) * LD + r0 + lo], x[s], acc);
+        return acc;
+    };
+    auto both = [&](int r0, int c0, int d0, typename MM::acc_t acc) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) a[u] += c * sl[(j0 + 8 * u) * NB + k];
-        }
-        // (step 2's reads of st ended at the barrier before this step)
+        for (int s = 0; s < 4; ++s)
+            acc = MM::mma(sl[(c0 + MM::kmap(kk, s)) * LD + r0 + lo], sl[(d0 + lo) * LD + c0 + MM::kmap(kk, s)], acc);
+        return acc;
+    };
+    auto put = [&](int r0, int c0, const typename MM::acc_t &v) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) st[(j0 + 8 * u) * 32 + i] = a[u];
-        __syncthreads();  // st complete; Q read by every lane
-#pragma unroll
-        for (int u = 0; u < 4; ++u) a[u] = T(0);
-#pragma unroll
-        for (int k = 0; k < 32; ++k) {
-            const T c = sl[(32 + k) * NB + 32 + i];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) a[u] += c * st[(j0 + 8 * u) * 32 + k];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) sl[(j0 + 8 * u) * NB + 32 + i] = -a[u];
+        for (int s = 0; s < 4; ++s) sl[(c0 + lo) * LD + r0 + MM::kmap(kk, s)] = -v[s];
+    };
+    const typename MM::acc_t zero = {T(0), T(0), T(0), T(0)};
+    // 2. two 32-blocks, wave p: C_p <- -inv(D_2p+1) C_p inv(D_2p)
+    if (wv < 2) {
+        const int o = 32 * wv;
+        const typename MM::acc_t x = both(o + 16, o, o, zero);
+        put(o + 16, o, left(o + 16, o + 16, x, zero));
     }
     __syncthreads();
+    // 3. the 64-block: Q <- -inv(R) Q inv(P), wave b a 16-column half of Q
+    if (wv < 2) {
+        const int c = 16 * wv;
+        typename MM::acc_t x0 = zero, x1 = zero;
+        if (wv == 0) {
+            x0 = both(32, 0, 0, x0);
+            x1 = both(48, 0, 0, x1);
+        }
+        x0 = both(32, 16, c, x0);
+        x1 = both(48, 16, c, x1);
+        const typename MM::acc_t y0 = left(32, 32, x0, zero);
+        const typename MM::acc_t y1 = left(48, 48, x1, left(48, 32, x0, zero));
+        __builtin_amdgcn_sched_barrier(0);
+        step3[0] = y0;
+        step3[1] = y1;
+    }
+    __syncthreads();  // Q read by both waves
+    if (wv < 2) {
+        put(32, 16 * wv, step3[0]);
+        put(48, 16 * wv, step3[1]);
+    }
+    __syncthreads();
+    // write: column-major 64 x 64; an upper block's inverse is J inv(L) J
+    T *w = W + blk * NB * NB;
+#pragma unroll 8
+    for (int e = t; e < NB * NB; e += NT) {
+        int i = e % NB, j = e / NB;  // element (i, j) of the stored inverse
+        T val;
+        if (lower || i >= nb || j >= nb)
+            val = (i < nb && j < nb) || lower ? sl[j * LD + i] : (i == j ? T(1) : T(0));
+        else
+            val = sl[(nb - 1 - j) * LD + (nb - 1 - i)];
+        w[e] = val;
+    }
     // Condition of the block, kappa_1 = ||L||_1 ||inv(L)||_1 (both exact, the
     // inverse being in LDS): an explicitly inverted block applied as a
     // product has backward error growing with kappa * u, so a block above
     // LEAF_REFINE_KAPPA is flagged and the panels follow its product with
     // one step of refinement (X += inv(L) (B - L X)).
-    if (F != nullptr && t < NB) {
-        T ni = T(0);
-#pragma unroll 8
-        for (int i = 0; i < NB; ++i) {
-            const T a = sl[t * NB + ((i + t) & (NB - 1))];
-            ni += a < T(0) ? -a : a;
+    if (F != nullptr) {
+        partial_sums(sp + 256);
+        __syncthreads();
+        if (t < 64) {
+            T nl = sp[t] + sp[t + 64] + sp[t + 128] + sp[t + 192];
+            T ni = sp[t + 256] + sp[t + 320] + sp[t + 384] + sp[t + 448];
+            for (int o = 32; o > 0; o >>= 1) {
+                const T l = __shfl_xor(nl, o), i = __shfl_xor(ni, o);
+                nl = l > nl ? l : nl;
+                ni = i > ni ? i : ni;
+            }
+            if (t == 0) {
+                const T kappa = nl * ni;
+                F[blk] = (kappa > T(LEAF_REFINE_KAPPA) || !(kappa == kappa)) ? 1 : 0;
+            }
         }
-        for (int o = 32; o > 0; o >>= 1) {
-            const T other = __shfl_xor(ni, o);
-            ni = other > ni ? other : ni;
-        }
-        if (t == 0) {
-            const T kappa = nl * ni;
-            F[blk] = (kappa > T(LEAF_REFINE_KAPPA) || !(kappa == kappa)) ? 1 : 0;
-        }
-    }
-    // write: column-major 64 x 64; an upper block's inverse is J inv(L) J
-    T *w = W + blk * NB * NB;
-#pragma unroll 4
-    for (int e = t; e < NB * NB; e += NT) {
-        int i = e % NB, j = e / NB;  // element (i, j) of the stored inverse
-        T val;
-        if (lower || i >= nb || j >= nb)
-            val = (i < nb && j < nb) || lower ? sl[j * NB + i] : (i == j ? T(1) : T(0));
-        else
-            val = sl[(nb - 1 - j) * NB + (nb - 1 - i)];
-        w[e] = val;
     }
 }
 
@@ -390,17 +431,17 @@ __global__ __launch_bounds__(LEAF_COLS) void trtri_kernel(int64_t n, const T *__
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void trtri64_kernel(int64_t n, const T *__restrict__ A, int64_t rs, int64_t cs,
                                                       int lower, int unit, T *__restrict__ W, int *__restrict__ F) {
-    __shared__ __attribute__((aligned(16))) T sl[64 * 64];
-    __shared__ __attribute__((aligned(16))) T st[32 * 32];
-    trtri64_block<T>(n, blockIdx.x, A, rs, cs, lower != 0, unit != 0, W, sl, st, F);
+    __shared__ __attribute__((aligned(16))) T sl[64 * TRTRI_LD];
+    __shared__ T sp[TRTRI_SP];
+    trtri64_block<T>(n, blockIdx.x, A, rs, cs, lower != 0, unit != 0, W, sl, sp, F);
 }
 
 // Batched form: one work-group per (system, block) pair.
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void batch_trtri_kernel(const BatchSys<T> *__restrict__ sys,
                                                          const int2 *__restrict__ blk) {
-    __shared__ __attribute__((aligned(16))) T sl[64 * 64];
-    __shared__ __attribute__((aligned(16))) T st[32 * 32];
+    __shared__ __attribute__((aligned(16))) T sl[64 * TRTRI_LD];
+    __shared__ T sp[TRTRI_SP];
     const int2 b = blk[blockIdx.x];
     const BatchSys<T> &S = sys[b.x];
     // the diagonal blocks of the effective matrix in its natural orientation:
@@ -409,7 +450,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void b
     const bool right = (S.wrs != 1);
     const int64_t rs = right ? S.mcs : S.mrs, cs = right ? S.mrs : S.mcs;
     const bool lower = right ? (S.lower == 0) : (S.lower != 0);
-    trtri64_block<T>(S.n, b.y, S.M, rs, cs, lower, false, (T *)S.W, sl, st, (int *)S.F);
+    trtri64_block<T>(S.n, b.y, S.M, rs, cs, lower, false, (T *)S.W, sl, sp, (int *)S.F);
 }
 
 template <typename T>
