@@ -16,6 +16,7 @@
 // caller's stream; pivots and info stay on the device.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <limits>
 #include <mutex>
 #include <type_traits>
@@ -702,64 +703,115 @@ __global__ void laswp_kernel(int64_t ncols, T *__restrict__ A, int64_t lda, int6
 
 // The same interchanges as one row permutation, for blocks whose rows fit
 // the work-group's LDS.  Positions are taken relative to b = k1 - 1; swap k
-// (0-based) exchanges positions k and p_k >= k.  Every work-group composes
-// the K swaps into src (the final content of position x is the old content
-// of position src[x]) with one thread walking them in LDS, lists the
-// positions past K that the swaps moved, and then permutes its columns: each
-// thread loads up to LASWP_R moved entries of a column, a barrier, and the
-// stores.  The sequential part runs at LDS latency instead of one dependent
-// round trip to memory per swap and column.
-constexpr int LASWP_THREADS = 1024, LASWP_R = 16;
-constexpr int LASWP_LDS = 40960 - 64;  // ints: src map (span) + pivots / moved list (K)
+// (0-based) exchanges positions k and p_k >= k.  Every work-group finds where
+// each final row comes from and then permutes its columns.
+//
+// What was at position q before swap k came there with the latest earlier
+// swap j that targets q (from position j before swap j), or was there from
+// the start.  So every position's source is a short walk of its own over
+// lists of the swaps that target a position, all positions at once: composing
+// the swaps in order, one LDS round trip each, took 0.1 us per swap (430 us
+// for the 4096 of a half of n = 8192, 6 of LU's 43 ms there).  Then every
+// thread moves up to LASWP_R entries at a time, several columns per pass where
+// few rows move: all loads, a barrier, the stores.
+constexpr int LASWP_THREADS = 1024, LASWP_R = 16, LASWP_COLS = 4;
+constexpr int LASWP_LDS = 163840 - 64;  // bytes: 4 per row of the block, 10 per swap
+constexpr int LASWP_SPAN = 38912;       // rows (a source is 16 bits, and LDS holds 812 swaps beside them)
+// swaps of one launch over span rows
+inline int64_t laswp_swaps(int64_t span) {
+    const int64_t k = (LASWP_LDS - 4 * span) / 10 / 2 * 2, most = LASWP_R * LASWP_THREADS / 2;
+    return k < most ? k : most;
+}
 
 template <typename T>
 __global__ __launch_bounds__(LASWP_THREADS) void laswp_perm_kernel(int64_t ncols, T *__restrict__ A, int64_t lda,
                                                                    int64_t b, int K, int span,
                                                                    const int64_t *__restrict__ ipiv, int64_t r0) {
-    __shared__ int s_map[LASWP_LDS];
+    __shared__ __attribute__((aligned(4))) char s_mem[LASWP_LDS];
     __shared__ int s_moved;
-    int *src = s_map, *lst = s_map + span;
+    int *head = reinterpret_cast<int *>(s_mem);                      // position -> a swap that targets it, -1 none
+    uint16_t *piv = reinterpret_cast<uint16_t *>(s_mem + 4 * span);  // swap -> its target
+    uint16_t *next = piv + K;                                        // swap -> another with the same target
+    uint16_t *src = next + K;                                        // position < K -> the row that ends there
+    uint16_t *dst = src + K, *dsrc = dst + K;                        // rows past K that move, and their sources
     const int t = threadIdx.x;
-    for (int x = t; x < span; x += LASWP_THREADS) src[x] = x;
-    for (int k = t; k < K; k += LASWP_THREADS) {
-        const int64_t p = ipiv[b + k] - 1 - r0 - b;
-        lst[k] = (p >= k && p < span) ? (int)p : k;  // pivots lie in [k, span)
-    }
+    constexpr uint16_t NONE = 0xffff;
+    for (int x = t; x < span; x += LASWP_THREADS) head[x] = -1;
     if (t == 0) s_moved = 0;
     __syncthreads();
-    if (t == 0) {
-        for (int k = 0; k < K; ++k) {
-            const int p = lst[k];
-            if (p != k) {
-                const int u = src[k];
-                src[k] = src[p];
-                src[p] = u;
+    for (int k = t; k < K; k += LASWP_THREADS) {
+        const int64_t q = ipiv[b + k] - 1 - r0 - b;
+        const int p = (q >= k && q < span) ? (int)q : k;  // pivots lie in [k, span)
+        piv[k] = (uint16_t)p;
+        const int old = atomicExch(&head[p], k);
+        next[k] = old < 0 ? NONE : (uint16_t)old;
+    }
+    __syncthreads();
+    // the row at position q before swap k
+    auto source = [&](int q, int k) {
+        for (;;) {
+            int j = -1;
+            for (int c = head[q]; c >= 0;) {
+                if (c < k && c > j) j = c;
+                const uint16_t n = next[c];
+                c = n == NONE ? -1 : (int)n;
+            }
+            if (j < 0) return q;
+            q = j;
+            k = j;
+        }
+    };
+    for (int x = t; x < span; x += LASWP_THREADS) {
+        if (x < K) {
+            src[x] = (uint16_t)source(piv[x], x);
+        } else if (head[x] >= 0) {
+            const int from = source(x, K);
+            if (from != x) {
+                const int at = atomicAdd(&s_moved, 1);
+                dst[at] = (uint16_t)x;
+                dsrc[at] = (uint16_t)from;
             }
         }
     }
     __syncthreads();
-    // positions past K hold their own rows unless a swap moved them
-    for (int x = K + t; x < span; x += LASWP_THREADS)
-        if (src[x] != x) lst[atomicAdd(&s_moved, 1)] = x;
-    __syncthreads();
     const int tot = K + s_moved;
+    auto to = [&](int i) { return i < K ? i : (int)dst[i - K]; };
+    auto from = [&](int i) { return i < K ? (int)src[i] : (int)dsrc[i - K]; };
+    if (tot <= LASWP_THREADS) {
+        const int w = (tot + 63) / 64 * 64, cpp = LASWP_THREADS / w;  // threads per column, columns side by side
+        const int i = t % w, side = t / w;
+        const bool on = side < cpp && i < tot;
+        const int x = on ? to(i) : 0, y = on ? from(i) : 0;
+        const bool move = on && x != y;
+        for (int64_t c0 = (int64_t)blockIdx.x * cpp * LASWP_COLS; c0 < ncols; c0 += (int64_t)gridDim.x * cpp * LASWP_COLS) {
+            T v[LASWP_COLS];
+#pragma unroll
+            for (int u = 0; u < LASWP_COLS; ++u) {
+                const int64_t c = c0 + u * cpp + side;
+                v[u] = move && c < ncols ? A[c * lda + b + y] : T(0);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < LASWP_COLS; ++u) {
+                const int64_t c = c0 + u * cpp + side;
+                if (move && c < ncols) A[c * lda + b + x] = v[u];
+            }
+        }
+        return;
+    }
     for (int64_t c = blockIdx.x; c < ncols; c += gridDim.x) {
         T *col = A + c * lda + b;
         T v[LASWP_R];
 #pragma unroll
         for (int r = 0; r < LASWP_R; ++r) {
             const int i = t + r * LASWP_THREADS;
-            const int x = i < K ? i : (i < tot ? lst[i - K] : 0);
-            v[r] = (i < tot) ? col[src[x]] : T(0);
+            v[r] = (i < tot) ? col[from(i)] : T(0);
         }
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < LASWP_R; ++r) {
             const int i = t + r * LASWP_THREADS;
-            if (i < tot) {
-                const int x = i < K ? i : lst[i - K];
-                if (src[x] != x) col[x] = v[r];
-            }
+            if (i < tot && from(i) != to(i)) col[to(i)] = v[r];
         }
     }
 }
@@ -875,20 +927,26 @@ struct LuRec {
         return st == NLA_OK;
     }
 
-    // interchanges k1..k2 of the m-row block at A on ncols columns: the LDS
-    // permutation when its map fits, else the sequential walk
+    // interchanges k1..k2 of the m-row block at A on ncols columns: as
+    // permutations of what fits LDS, else the sequential walk
     void laswp(T *A, int64_t m, int64_t ncols, int64_t k1, int64_t k2, const int64_t *ipiv, int64_t r0) {
-        if (ncols <= 0 || k2 < k1 || st != NLA_OK) return;
-        const int64_t K = k2 - k1 + 1, b = k1 - 1, span = m - b;
-        if (2 * K <= (int64_t)LASWP_R * LASWP_THREADS && span + K <= LASWP_LDS) {
-            const unsigned g = (unsigned)(ncols < 256 ? ncols : 256);
+        if (ncols <= 0) return;
+        while (k1 <= k2 && st == NLA_OK) {
+            const int64_t b = k1 - 1, span = m - b;
+            if (span > LASWP_SPAN) {
+                hipLaunchKernelGGL(laswp_kernel<T>, dim3((unsigned)((ncols + 63) / 64)), dim3(64), 0, s, ncols, A, lda,
+                                   k1, k2, ipiv, r0);
+                ok(hipGetLastError(), "laswp");
+                return;
+            }
+            const int64_t K = std::min(k2 - b, laswp_swaps(span));
+            const int64_t per = K <= LASWP_THREADS / 2 ? LASWP_THREADS / (2 * K) * LASWP_COLS : 1;  // columns of a pass
+            const unsigned g = (unsigned)std::min<int64_t>((ncols + per - 1) / per, 512);
             hipLaunchKernelGGL(laswp_perm_kernel<T>, dim3(g), dim3(LASWP_THREADS), 0, s, ncols, A, lda, b, (int)K,
                                (int)span, ipiv, r0);
-        } else {
-            hipLaunchKernelGGL(laswp_kernel<T>, dim3((unsigned)((ncols + 63) / 64)), dim3(64), 0, s, ncols, A, lda, k1,
-                               k2, ipiv, r0);
+            ok(hipGetLastError(), "laswp");
+            k1 += K;
         }
-        ok(hipGetLastError(), "laswp");
     }
 
     // Factor the m x n block at A, whose first row and column are the global

@@ -1103,7 +1103,10 @@ hipError_t launch_panel(const PanelArgs<T> &a, hipStream_t s) {
     // 37.8 / 23.8, 45.5 / 30.8, 72.6 / 59.8, 128 rows 6.7 / 5.8 and with 8192
     // columns 11.2 / 12.2; FP32 TRSM 512 rows 27.6 / 22.9, 30.9 / 26.1,
     // 46.6 / 49.7, TRMM 27.1 / 17.9, 30.1 / 22.3, 47.7 / 43.8.
-    const bool many = a.m > 16 * 256, small = a.nbig <= 128;
+    // A unit diagonal is LU's: its blocks are as often flagged for refinement
+    // as not, which the eight waves do on MFMA (in the LU of n = 8192, left-looking /
+    // eight waves: 64 rows 25 / 8 us, 128 rows 48 / 15).
+    const bool many = a.m > 16 * 256, small = a.nbig <= 128 && !a.unit;
     if (a.nbig > PU_MAX || a.waves == 4 || (a.waves == 0 && (a.trmm ? many && small : many || small)))
         return a.trmm ? launch_panel_left_n<T, true>(a, s) : launch_panel_left_n<T, false>(a, s);
     return a.strip == 32 ? launch_panel_w<T, 32>(a, s) : launch_panel_w<T, 16>(a, s);

@@ -254,3 +254,26 @@ def test_register_panel_edges(nla, split_rows, dtype, m, n):
     assert torch.equal(p1, p2)
     tol = 1e-12 if dtype == torch.float64 else 1e-5
     assert torch.max(torch.abs(L1 - L2)).item() <= tol * torch.max(torch.abs(L1)).item()
+
+
+@pytest.mark.parametrize("m,n", [(5000, 5000), (32768, 6656), (38913, 1300)])
+def test_interchanges_large(nla, m, n):
+    """Interchanges of whole halves at once, in several permutations of one
+    block (32768 rows leave room for 3270 swaps at a time) and past the rows a
+    permutation takes: P*A = L*U on sampled columns, in float64 (the residual
+    of one factorization: a few n eps of |L||U|)."""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m)
+    A0 = torch.empty((n, m), dtype=torch.float64, device=DEV).normal_(generator=g).t()
+    LU, ipiv, info = nla.getrf2_(A0.clone())
+    assert info == 0
+    p = np.arange(m)
+    for i, j in enumerate(ipiv.cpu().numpy() - 1):
+        p[i], p[j] = p[j], p[i]
+    cols = torch.tensor([0, 63, 64, n // 2, n - 1], device=DEV)
+    L = torch.tril(LU, -1)
+    L.diagonal().fill_(1.0)
+    U = torch.triu(LU[:n])[:, cols]
+    err = L @ U - A0[:, cols][torch.from_numpy(p).to(DEV)]
+    bound = 4 * n * 2.2e-16 * (L.abs() @ U.abs())
+    assert torch.all(err.abs() <= bound)
