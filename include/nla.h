@@ -562,12 +562,14 @@ int32_t nla_serve_destroy(nla_server server);
  *                      one fused panel launch (default, needs leaf mode 1),
  *                      0 = recurse to 64-leaves;
  *   NLA_CFG_PANEL_ROWS_F32 / _F64: panel size for that dtype, a multiple of
- *                      64 in [64, 1024], or 0 (default): by layout, 512
- *                      where the panel's rows are contiguous (left side
- *                      with trans 'N', right side with 'T'), else 256;
+ *                      64 in [64, 1024], or 0 (default): by shape, 512,
+ *                      but 256 for an FP64 TRSM with up to 2048 columns
+ *                      whose panel rows are not contiguous (left side with
+ *                      trans 'T', right side with 'N');
  *                      above 512 rows FP64 panels use 16 columns per group;
  *   NLA_CFG_PANEL_STRIP_F32 / _F64: right-hand-side columns per panel
- *                      work-group, 16 (default) or 32;
+ *                      work-group, 16 (default; eight-wave panels take
+ *                      32 where there are more than 4096) or 32;
  *   NLA_CFG_PANEL_WAVES: waves per panel work-group (panels up to 512 rows):
  *                      4 (left-looking, 16 columns, two and more groups per
  *                      CU) or 8 (32-row units, right-looking TRSM); 0

@@ -112,16 +112,21 @@ static std::atomic<int> g_leaf_mode{-1};
 static std::atomic<int> g_panel{-1};
 // Panel shape per dtype (index NLA_F32 / NLA_F64): the largest diagonal
 // block handed to one fused panel launch (a multiple of 64, <= PANEL_MAX,
-// or 0: by layout) and its RHS columns per work-group.  By layout: where the
-// panel's rows are contiguous in memory (left side with op(A) = A, right
-// side with op(A) = A^T) its fragment loads are coalesced and 512 rows win;
-// otherwise every fragment element is its own cache line and 256 rows
-// win.  Measured on MI355X at n = 8192, 4 waves (rows 256 / 512): FP32 TRSM
-// L-L-N 5.06 / 4.83 ms, R-L-T 5.48 / 5.17, L-L-T 5.49 / 6.06, R-L-N
-// 5.84 / 6.33; FP64 TRSM L-L-N 9.39 / 9.10, L-L-T 9.89 / 10.10, R-L-N
-// 10.08 / 10.19; FP64 TRMM L-L-T 9.96 / 10.22.  16 columns for both dtypes.
+// or 0: by shape) and the least RHS columns per work-group (16 or 32,
+// launch_panel).  By shape: 512 rows, but 256 where the rows of an FP64 TRSM
+// panel are not contiguous in memory (left side with op(A) = A^T, right side
+// with op(A) = A: every fragment element is a load of its own) and there are
+// few columns, so that the chain of one 512-row panel is not hidden.
+// Measured on MI355X at n = 2048, rows 256 / 512 (us): FP64 TRSM L-L-T with
+// 64 / 1024 / 3000 / 4096 / 8192 columns 217 / 232, 285 / 298, 519 / 484,
+// 547 / 490, 966 / 833; FP32 TRSM 143 / 134, 173 / 163, 267 / 236, 276 / 251,
+// 543 / 423; FP64 TRMM 188 / 190, 264 / 258, 508 / 446, 531 / 447, 889 / 663.
+// With contiguous rows 512 wins throughout (FP64 TRSM L-L-N 188 / 181,
+// 254 / 241, 419 / 377, 481 / 411, 843 / 748).
 static std::atomic<int> g_panel_rows[2] = {{0}, {0}};
-static int panel_rows_default(bool contiguous) { return contiguous ? 512 : 256; }
+static int panel_rows_default(bool trsm64, bool contiguous, int64_t m) {
+    return trsm64 && !contiguous && m <= 2048 ? 256 : 512;
+}
 static std::atomic<int> g_panel_strip[2] = {{PANEL_STRIP}, {PANEL_STRIP}};
 // Waves per panel work-group: 4, 8, or 0 = by the panel's shape (launch_panel).
 static std::atomic<int> g_panel_waves{0};
@@ -544,7 +549,7 @@ static int32_t rectrxm_typed(char side, char uplo, char trans, char func, double
         const int pr = g_panel_rows[di].load();
         // the panel's row stride: A's for the left side, its transpose's for the right
         const bool contiguous = (side == 'L' ? A.rs : A.cs) == 1;
-        r.panel_rows = pr ? pr : panel_rows_default(contiguous);
+        r.panel_rows = pr ? pr : panel_rows_default(func == 'S' && di == NLA_F64, contiguous, m);
         r.panel_strip = g_panel_strip[di].load();
         r.panel_waves = g_panel_waves.load();
     }

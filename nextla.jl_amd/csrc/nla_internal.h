@@ -53,7 +53,7 @@ struct LeafArgs {
 };
 
 // Largest diagonal block the fused panel kernel solves in one launch, and the
-// default RHS columns per work-group (16 or 32 per launch).
+// default of the least RHS columns per work-group (16 or 32 per launch).
 constexpr int PANEL_MAX = 1024;
 constexpr int PANEL_STRIP = 16;
 
@@ -75,7 +75,7 @@ struct PanelArgs {
     // TRSM: per 64-block flags from launch_trtri_blocks (nullable): a flagged
     // block's product with its inverse is followed by one refinement step
     const int *F = nullptr;
-    int strip = PANEL_STRIP;  // RHS columns per work-group: 16 or 32
+    int strip = PANEL_STRIP;  // least RHS columns per work-group: 16 or 32
     bool unit = false;        // unit diagonal (taken as 1, not read)
     int waves = 0;            // waves per work-group up to 512 rows: 4, 8, or 0 by shape
     // TRSM, fp32: *xmax = max(*xmax, max |X|) over the panel's solution (a

@@ -923,6 +923,7 @@ __device__ __forceinline__ void panel_trmm(int nbig, int64_t m, int64_t c0, cons
         const int r0 = 32 * u;
         PanelAcc<T, 2, CBW> acc;
         acc.zero();
+        T sum[2][CBW][4] = {};
         // off the diagonal, whole 32-deep pieces: [ka, kb); an upper unit's last one may be short
         const int ka = lower ? 0 : r0 + 32, kb = lower ? r0 : nbig, np = (kb - ka) / 32;
         PR rows;
@@ -962,6 +963,16 @@ __device__ __forceinline__ void panel_trmm(int nbig, int64_t m, int64_t c0, cons
                     rows.load(ka + 32 * (nx < np ? nx : np - 1), f[(v + PD - 1) % PD]);
                     panel_mul<T, CBW, 2>(f[v], xb + ka + 32 * (i + v), LDB, acc);
                 }
+                // sums of 96 products at a time: one chain along 512 rows
+                // would round more than the 256-row panels and their updates
+                // (FP32 R-U-N n = 4096: 3.0e-7 of the result against 2.1e-7)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int cb = 0; cb < CBW; ++cb)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) sum[b][cb][e] += acc.at(b, cb, e);
+                acc.zero();
             }
 #pragma unroll
             for (int v = 0; v < PD - 1; ++v)
@@ -982,7 +993,7 @@ __device__ __forceinline__ void panel_trmm(int nbig, int64_t m, int64_t c0, cons
                 for (int e = 0; e < 4; ++e) {
                     const int c = cb * 16 + MF::di(lane, e);
                     if (r < nbig && c < ncol) {
-                        const T v = unit ? acc.at(b, cb, e) + bs[c * LDB + r] : acc.at(b, cb, e);
+                        const T x = sum[b][cb][e] + acc.at(b, cb, e), v = unit ? x + bs[c * LDB + r] : x;
                         B[r * brs + c * bcs] = v * scale;
                     }
                 }
@@ -1096,20 +1107,28 @@ hipError_t launch_panel(const PanelArgs<T> &a, hipStream_t s) {
     if (a.nbig > PANEL_MAX) return hipErrorInvalidValue;
     if (a.strip != 16 && a.strip != 32) return hipErrorInvalidValue;
     // Four waves and 16 columns leave room for two and more work-groups on a
-    // CU: the left-looking strip wins where there are more strips than CUs, or
-    // no chain to shorten.  Measured on MI355X (us, left / eight waves): FP64
+    // CU: the left-looking strip wins where a TRSM has more strips than CUs and
+    // M's columns are contiguous (along k it loads one element per cache line),
+    // or where there is no chain to shorten.  Otherwise, more strips
+    // than CUs take 32 columns a group, which halves the reads of M.  Measured on MI355X (us, left / eight waves): FP64
     // TRSM of 512 rows with 64 / 4096 / 8192 columns 40.2 / 32.8, 47.9 / 41.0,
     // 75.0 / 80.8, 128 rows 7.0 / 7.5, 64 rows 4.4 / 4.5; FP64 TRMM 512 rows
     // 37.8 / 23.8, 45.5 / 30.8, 72.6 / 59.8, 128 rows 6.7 / 5.8 and with 8192
     // columns 11.2 / 12.2; FP32 TRSM 512 rows 27.6 / 22.9, 30.9 / 26.1,
-    // 46.6 / 49.7, TRMM 27.1 / 17.9, 30.1 / 22.3, 47.7 / 43.8.
+    // 46.6 / 49.7, TRMM 27.1 / 17.9, 30.1 / 22.3, 47.7 / 43.8.  Whole calls of
+    // n = 2048 with 8192 columns (left / eight waves of 16 / of 32 columns):
+    // FP64 TRSM L-L-N 748 / 770 / 805, L-L-T 961 / 860 / 833, FP32 L-L-N
+    // 434 / 450 / 435, L-L-T 685 / 446 / 423; FP64 TRMM L-L-N 719 / 669 / 646,
+    // L-L-T 977 / 777 / 663, FP32 421 / 406 / 394, 720 / 396 / 371; with 3000
+    // columns 16 win throughout (FP64 L-L-T 484 / 645, TRMM 446 / 492).
     // A unit diagonal is LU's: its blocks are as often flagged for refinement
     // as not, which the eight waves do on MFMA (in the LU of n = 8192, left-looking /
     // eight waves: 64 rows 25 / 8 us, 128 rows 48 / 15).
-    const bool many = a.m > 16 * 256, small = a.nbig <= 128 && !a.unit;
-    if (a.nbig > PU_MAX || a.waves == 4 || (a.waves == 0 && (a.trmm ? many && small : many || small)))
+    const bool many = a.m > 16 * 256, small = a.nbig <= 128 && !a.unit, left = a.trmm ? many && small
+                                                                                      : (many && a.mrs == 1) || small;
+    if (a.nbig > PU_MAX || a.waves == 4 || (a.waves == 0 && a.strip != 32 && left))
         return a.trmm ? launch_panel_left_n<T, true>(a, s) : launch_panel_left_n<T, false>(a, s);
-    return a.strip == 32 ? launch_panel_w<T, 32>(a, s) : launch_panel_w<T, 16>(a, s);
+    return a.strip == 32 || many ? launch_panel_w<T, 32>(a, s) : launch_panel_w<T, 16>(a, s);
 }
 
 template hipError_t launch_panel<float>(const PanelArgs<float> &, hipStream_t);

@@ -381,3 +381,21 @@ def test_eight_wave_panels(nla, dt, n):
     finally:
         _lib.set_config(_lib.NLA_CFG_PANEL_WAVES, old_w)
         _lib.set_config(rows_key, old_r)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [129, 500, 640])
+@pytest.mark.parametrize("m", [2049, 4097, 4113])
+def test_panels_many_columns(nla, dt, n, m):
+    """The default panels where they change with the columns (256 or 512 rows
+    past 2048, 32 columns per group or the left-looking strip past 4096), with
+    a ragged last strip: the oracle's bounds."""
+    rng = np.random.default_rng(n + m)
+    for side, uplo, trans, func in itertools.product("LR", "LU", "NT", "SM"):
+        T = np.tril(rng.uniform(-1, 1, (n, n)) / np.sqrt(n), -1)
+        np.fill_diagonal(T, 2 + rng.random(n))
+        A = np.asfortranarray((T if uplo == "L" else T.T).astype(dt))
+        B = rng.standard_normal((n, m) if side == "L" else (m, n)).astype(dt)
+        Ad, Bd = (torch.from_numpy(np.ascontiguousarray(t.T)).cuda().t() for t in (A, B))
+        nla.unified_rectrxm_(side, uplo, trans, 1.5, func, Ad, Bd)
+        check_bound(side, uplo, trans, 1.5, func, A, B, Bd.cpu().numpy())
