@@ -242,40 +242,106 @@ __device__ __forceinline__ void gemm_tile(int64_t M, int64_t N, int64_t K, T alp
         ly.store(lds_y[buf], t);
     };
     const int lo = lane % MF::BD, lk = lane / MF::BD;
-    auto multiply = [&](int buf) {
+    // One k step from one stage of LDS, and a part of one: the operands of a
+    // single depth into registers, and their products.
+    constexpr int KS = BK / MF::KD;
+    auto read = [&](int buf, int ks, T *a, T *b) {
         const NLA_LDS T *sx = lds_x[buf];
         const NLA_LDS T *sy = lds_y[buf];
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) a[cb] = LY::at(sy, wn * TWN + cb * MF::BD + lo, ks * MF::KD + lk);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) b[rb] = LX::at(sx, wm * TWM + rb * MF::BD + lo, ks * MF::KD + lk);
+    };
+    auto products = [&](const T *a, const T *b) {
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) acc[cb][rb] = MF::mma(a[cb], b[rb], acc[cb][rb]);
+    };
+    T a[2][CB], b[2][RB];
+    auto multiply = [&](int buf) {
         __builtin_amdgcn_s_setprio(1);  // issue priority to waves in their MFMA cluster
 #pragma unroll
-        for (int ks = 0; ks < BK; ks += MF::KD) {
+        for (int ks = 0; ks < KS; ++ks) {
             T a[CB], b[RB];
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb) a[cb] = LY::at(sy, wn * TWN + cb * MF::BD + lo, ks + lk);
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) b[rb] = LX::at(sx, wm * TWM + rb * MF::BD + lo, ks + lk);
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb) acc[cb][rb] = MF::mma(a[cb], b[rb], acc[cb][rb]);
+            read(buf, ks, a, b);
+            products(a, b);
         }
         __builtin_amdgcn_s_setprio(0);
     };
-    // whole steps, the next one's loads in flight behind the products
-    if (nfull > 0) {
-        lx.load(0);
-        ly.load(0);
-        stage(0, 0);
-    }
-    __syncthreads();
-    for (int kt = 0; kt < nfull; ++kt) {
-        const int cur = kt & 1;
-        const bool more = kt + 1 < nfull;
-        if (more) {
-            lx.load(kt + 1);
-            ly.load(kt + 1);
+    // Whole steps.  The waves of a work-group reach the end of a step together,
+    // so what stands there idles the matrix cores: with the LDS stores, the
+    // barrier and the first LDS reads in a row that was 4 to 8 % of the FP64
+    // loop.  So the operands of a depth are read ahead of the products before
+    // it, the next step's stores stand among the products (its loads were
+    // issued a whole step before), and the barrier comes before the last
+    // products, which cover the next step's first reads.  Measured on MI355X
+    // (us, before / after): FP64 4096 x 8192 x 4096 4128 / 4016, 2048 x 2048 x
+    // 1024 151 / 143, 3000^3 1217 / 1158; FP32 1531 x 1023 x 976 44.1 / 43.0.
+    // Sixteen waves (FP32 256 x 256) have 128 registers each, too few for two
+    // sets of operands (2023 / 2273 at 4096 x 8192 x 4096), and keep the plain
+    // order.
+    if constexpr (NT > 512) {
+        if (nfull > 0) {
+            lx.load(0);
+            ly.load(0);
+            stage(0, 0);
         }
-        multiply(cur);
-        if (more) stage(kt + 1, cur ^ 1);
+        __syncthreads();
+        for (int kt = 0; kt < nfull; ++kt) {
+            const int cur = kt & 1;
+            const bool more = kt + 1 < nfull;
+            if (more) {
+                lx.load(kt + 1);
+                ly.load(kt + 1);
+            }
+            multiply(cur);
+            if (more) stage(kt + 1, cur ^ 1);
+            __syncthreads();
+        }
+    } else {
+        static_assert(KS % 2 == 0, "every step starts with the same set");
+        auto ahead = [&](int of) {
+            __builtin_amdgcn_s_setprio(1);
+            products(a[of], b[of]);
+            __builtin_amdgcn_s_setprio(0);
+        };
+        if (nfull > 0) {
+            lx.load(0);
+            ly.load(0);
+            stage(0, 0);
+            lx.load(nfull > 1 ? 1 : 0);
+            ly.load(nfull > 1 ? 1 : 0);
+            __syncthreads();
+            read(0, 0, a[0], b[0]);
+            for (int kt = 0; kt + 1 < nfull; ++kt) {
+                const int cur = kt & 1;
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    const int to = (ks + 1) & 1;
+                    if (ks + 1 < KS) {
+                        read(cur, ks + 1, a[to], b[to]);
+                    } else {
+                        __syncthreads();
+                        read(cur ^ 1, 0, a[to], b[to]);
+                    }
+                    ahead(ks & 1);
+                    if (ks == KS - 2) {
+                        stage(kt + 1, cur ^ 1);
+                        const int next = kt + 2 < nfull ? kt + 2 : nfull - 1;
+                        lx.load(next);
+                        ly.load(next);
+                    }
+                }
+            }
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const int to = (ks + 1) & 1;
+                if (ks + 1 < KS) read((nfull - 1) & 1, ks + 1, a[to], b[to]);
+                ahead(ks & 1);
+            }
+        }
         __syncthreads();
     }
     // the checked ones (at most two), on their own: a choice of loads inside
@@ -288,7 +354,17 @@ __device__ __forceinline__ void gemm_tile(int64_t M, int64_t N, int64_t K, T alp
         ly.apply_bounds();
         stage(kt, kt & 1);
         __syncthreads();
-        multiply(kt & 1);
+        if constexpr (NT > 512) {
+            multiply(kt & 1);
+        } else {  // as in the loop: with multiply() here its registers fell worse (4032 / 4076 us at the first size)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                read(kt & 1, ks, a[0], b[0]);
+                __builtin_amdgcn_s_setprio(1);
+                products(a[0], b[0]);
+                __builtin_amdgcn_s_setprio(0);
+            }
+        }
         __syncthreads();
     }
 
