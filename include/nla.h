@@ -222,8 +222,8 @@ int32_t nla_trmm(char side, char uplo, char transa, char diag, int32_t dtype, do
  * block, applies its interchanges to the right block, solves
  * A12 = L11^-1·A12 with the unit-lower TRSM of this library (nla_trsm,
  * diag 'U'), updates A22 -= A21·A12 (nla_gemm), factors A22 and applies its
- * interchanges to the left block; a single column is one kernel (pivot =
- * first index of the largest |a|, swap, scale by the reciprocal).
+ * interchanges to the left block; a panel of up to 64 columns is one kernel
+ * (pivot = first index of the largest |a|, swap, scale by the reciprocal).
  *   A     m x n column-major (leading dimension lda), FP32 or FP64;
  *   ipiv  device array of min(m,n) int64: row i was interchanged with row
  *         ipiv[i] (1-based, as the reference);
@@ -582,20 +582,20 @@ int32_t nla_serve_destroy(nla_server server);
  *                      Bit 4 (0x10): systems above 512 rows are solved in
  *                      512-row stages (panels of the 512 class plus a grouped
  *                      GEMM) instead of as one 1024-row panel.
- *   NLA_CFG_LU_SPLIT_ROWS: nla_getrf2 leaves (blocks of up to 8 columns) of at
- *                      least this many rows are held in registers: one
- *                      work-group up to 4096 rows, above that one per 2048
- *                      rows up to 131072 rows (default 1: every leaf up to
- *                      that size; 0 = the one-work-group leaf that works in
- *                      global memory, for every size).
+ *   NLA_CFG_LU_SPLIT_ROWS: nla_getrf2 panels of at least this many rows are
+ *                      held in registers: one work-group up to 128 rows,
+ *                      above that up to 128 of them, to 131072 rows (default
+ *                      1: every panel up to that size; 0 = 8-column blocks
+ *                      in the one-work-group leaf that works in global
+ *                      memory, for every size).
  *   NLA_CFG_RESIDUAL:  residual of nla_rectrxm_mixed: NLA_RES_INT8 (default)
  *                      for n in [2048, 65536] and m >= 64, FP64 otherwise;
  *                      NLA_RES_FP64 for every size.  Read when the
  *                      workspace size is queried and when the solve starts
  *                      (the int8 residual needs the larger workspace).
- *   NLA_CFG_LU_SPIN_LIMIT: polls of a multi-work-group LU leaf's bounded
- *                      grid-barrier wait before it gives up (0 = default,
- *                      about a second).  A leaf whose wait runs out (its
+ *   NLA_CFG_LU_SPIN_LIMIT: polls of a multi-work-group LU panel's bounded
+ *                      wait before it gives up (0 = default, about a
+ *                      second).  A panel whose wait runs out (its
  *                      work-groups not all resident, e.g. beside another
  *                      persistent grid) is redone from a copy saved before
  *                      it by the one-work-group leaf, so nla_getrf2's result

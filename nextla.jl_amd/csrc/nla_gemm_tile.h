@@ -181,8 +181,7 @@ __device__ inline void tile_coords(int G, int g, int tiles_m, int &tm, int &tn) 
 }
 
 // One BM x BN tile of C at (row0, col0).  EDGE: the tile may reach past M or
-// N.  TRI: triangle mask (GemmArgs::tri), or 5: op(X) upper and op(Y) lower
-// (k >= row and k >= column: lauum's product).
+// N.  TRI: triangle mask (GemmArgs::tri).
 template <typename T, int BM, int BN, int BK, int WM, int WN, bool TX, bool TY, int TRI, bool EDGE>
 __device__ __forceinline__ void gemm_tile(int64_t M, int64_t N, int64_t K, T alpha, const T *__restrict__ X,
                                           int64_t ldx, const T *__restrict__ Y, int64_t ldy, T beta, T *C,
@@ -218,7 +217,6 @@ __device__ __forceinline__ void gemm_tile(int64_t M, int64_t N, int64_t K, T alp
     if (TRI == 2) kbeg = row0 < K ? row0 : K;
     if (TRI == 3) kbeg = col0 < K ? col0 : K;
     if (TRI == 4) kend = col0 + BN < K ? col0 + BN : K;
-    if (TRI == 5) kbeg = row0 > col0 ? row0 : col0;
     const int64_t kn = kend - kbeg, whole = EDGE ? kn - LX::VW : kn;
     const int nfull = whole > 0 ? (int)(whole / BK) : 0, nkt = (int)((kn + BK - 1) / BK);
 
@@ -234,8 +232,8 @@ __device__ __forceinline__ void gemm_tile(int64_t M, int64_t N, int64_t K, T alp
     auto stage = [&](int kt, int buf) {
         const int64_t k0 = kbeg + (int64_t)kt * BK;
         if (TRI == 1 && k0 + BK > row0) lx.template mask<true>(row0, k0, t);
-        if ((TRI == 2 || TRI == 5) && k0 < row0 + BM) lx.template mask<false>(row0, k0, t);
-        if ((TRI == 3 || TRI == 5) && k0 < col0 + BN) ly.template mask<false>(col0, k0, t);
+        if (TRI == 2 && k0 < row0 + BM) lx.template mask<false>(row0, k0, t);
+        if (TRI == 3 && k0 < col0 + BN) ly.template mask<false>(col0, k0, t);
         if (TRI == 4 && k0 + BK > col0) ly.template mask<true>(col0, k0, t);
         lx.store(lds_x[buf], t);
         __builtin_amdgcn_sched_barrier(0);  // the stores in the order of the loads: each waits for its own
