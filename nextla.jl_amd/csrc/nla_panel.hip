@@ -728,7 +728,12 @@ struct PanelSolve {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) fw[4 * q + e] = p[(16 * q + e) * wcs];
+            for (int e = 0; e < 4; ++e) fw[4 * q + e] = p[(inverse_col(q, e) - kk) * wcs];
+    }
+    // the inverse's columns in the order of their use (this lane's of the
+    // product e of block q): the diagonal block last, towards the diagonal
+    __device__ inline int inverse_col(int q, int e) const {
+        return 16 * ((wv + 1 + q) & 3) + (q < 3 ? kk + e : 4 * (lower ? e : 3 - e) + (kk >> 2));
     }
     __device__ inline int k_of(int s, int h) const { return 64 * block(s) + 32 * h; }
 
@@ -746,15 +751,22 @@ struct PanelSolve {
                     tmp[c * LDX + b0 + i] = r0 + i < nbig ? v : T(0);
                 }
     }
-    // x (+)= the inverse's row block times tmp
+    // x (+)= the inverse's row block times tmp, in one chain with the diagonal,
+    // which has the large terms, at its end: what comes after them is rounded
+    // at their size (512 x 512 FP32: 8.4e-8 L-L-N and 1.29e-7 L-L-T of the
+    // result in two chains of ascending k, 7.7e-8 and 8.3e-8 so).
     __device__ inline void apply_inverse(X &x) {
-        T g[1][8];
+        T v[CBW][16];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int cb = 0; cb < CBW; ++cb)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) g[0][e] = fw[8 * h + e];
-            panel_mul<T, CBW, 1>(g, tmp + lo * LDX + 32 * h + kk, LDX, x);
-        }
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[cb][4 * q + e] = tmp[(cb * 16 + lo) * LDX + inverse_col(q, e)];
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+#pragma unroll
+            for (int cb = 0; cb < CBW; ++cb) x.a[0][0][cb] = MF::mma(v[cb][e], fw[e], x.a[0][0][cb]);
     }
     __device__ inline void put_x(int s, const X &x) {
         const int r0 = 64 * block(s) + 16 * wv + lo;
