@@ -65,10 +65,13 @@ hipError_t launch_gemm(const GemmArgs<T> &a, hipStream_t s) {
     // smallest tile is 64 x 64: 512 x 512 x 256 9.2 / 5.4, 768 x 768 x 1024
     // 26.8 / 21.7, 1024 x 1024 x 256 10.2 / 11.8, 64 x 4096 x 4096 97 / 31,
     // 256 x 4096 x 4096 101 / 100.  Eight waves per tile, 64 x 16 and 64 x 64
-    // tiles were within 10 % of 32 x 32 with four or slower.
+    // tiles were within 10 % of 32 x 32 with four or slower.  FP64 with op(X)
+    // transposed, whose lanes load from 16 rows of memory, reaches 36 TFLOP/s
+    // here (48 otherwise): a block reflector of 8192 x 8192 with k = 256, 128
+    // tiles, takes 1453 / 1700 us tiled / split.
     if (a.leaf == 0 && a.tri == 0 && a.K > 0) {
         auto tiles = [&](int b) { return ((a.M + b - 1) / b) * ((a.N + b - 1) / b); };
-        const bool split = sizeof(T) == 8 ? tiles(128) <= (a.K < 128 ? 64 : 192) : tiles(64) <= 144;
+        const bool split = sizeof(T) == 8 ? tiles(128) <= (a.K < 128 ? 64 : (a.tx ? 96 : 192)) : tiles(64) <= 144;
         if (split) return launch_split<T, 2, 2, 4>(a, s);
     }
     return launch_gemm_tiled<T>(a, s);
