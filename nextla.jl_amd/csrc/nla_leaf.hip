@@ -226,19 +226,19 @@ __device__ __forceinline__ void trtri64_block(int64_t n, int64_t blk, const T *_
     if (F != nullptr) partial_sums(sp);
     // 1. inverses of the 16 x 16 diagonal blocks b: lane (b, c) solves D_b y =
     // e_c.  Each of its 16 quotients is a product with the reciprocal of the
-    // diagonal and one correction by the exact remainder (the quotient
-    // rounded, as a division gives it, in three dependent operations instead
-    // of a division's dozen); a block with an entry whose reciprocal or
+    // diagonal and one correction by the exact remainder (Markstein's step: the
+    // quotient rounded, as a division gives it, in three dependent operations
+    // instead of a division's dozen); a block with an entry whose reciprocal or
     // remainder could leave the normal range takes the divisions.
+    T x[16];
+    const int o1 = 16 * ((t & 63) >> 4), c1 = t & 15;
+    T *blk16 = sl + o1 * LD + o1;
     if (t < 64) {
         const T d = sl[t * LD + t], ad = fabs(d);
         constexpr T big = Mma16<T>::big, small = T(1) / big;
         const bool plain = __all(ad >= small && ad <= big);
         rinv[t] = T(1) / d;
-        T x[16];
-        const int o1 = 16 * (t >> 4), c1 = t & 15;
         __builtin_amdgcn_wave_barrier();
-        T *blk16 = sl + o1 * LD + o1;
 #pragma unroll
         for (int i = 0; i < 16; ++i) x[i] = (i == c1) ? T(1) : T(0);
         if (plain) {
@@ -258,7 +258,9 @@ __device__ __forceinline__ void trtri64_block(int64_t n, int64_t blk, const T *_
                 for (int r = j + 1; r < 16; ++r) x[r] -= blk16[j * LD + r] * x[j];
             }
         }
-        __builtin_amdgcn_wave_barrier();  // one wave, in order: every lane has read its block
+    }
+    __syncthreads();  // every lane has read its block, and every wave L for its column sums
+    if (t < 64) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) blk16[c1 * LD + i] = x[i];
     }
