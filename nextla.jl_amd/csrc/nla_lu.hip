@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <limits>
+#include <memory>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -849,26 +850,30 @@ __global__ void info_zero_kernel(int64_t *info) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *info = 0;
 }
 
-// Counters and published candidates of the split leaf, one buffer per
-// (device, stream): launches on one stream run in order, so they share it.
-struct SplitSync {
+// Exchange slots and saved block of the register panels, one buffer per
+// (device, stream): launches on one stream run in order, so they share it.  A
+// panel and the recovery launch that follows it are enqueued under the
+// buffer's lock: with another host thread's panel in between, the recovery
+// would find that panel's block saved.
+struct PanelSync {
     int dev;
     hipStream_t stream;
-    uint64_t *ptr;
+    uint64_t *ptr = nullptr;
+    std::mutex mu;
 };
 
-uint64_t *split_sync(hipStream_t s, int32_t *st) {
+PanelSync *panel_sync(hipStream_t s, int32_t *st) {
     static std::mutex mu;
-    static std::vector<SplitSync> cache;
+    static std::vector<std::unique_ptr<PanelSync>> cache;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) {
-        *st = report_hip(e, "lu split leaf device");
+        *st = report_hip(e, "lu panel device");
         return nullptr;
     }
     std::lock_guard<std::mutex> g(mu);
     for (auto &c : cache)
-        if (c.dev == dev && c.stream == s) return c.ptr;
+        if (c->dev == dev && c->stream == s) return c.get();
     uint64_t *p = nullptr;
     e = hipMalloc((void **)&p, SYNC_BYTES);
     if (e == hipSuccess) {
@@ -876,11 +881,14 @@ uint64_t *split_sync(hipStream_t s, int32_t *st) {
         e = hipGetLastError();
     }
     if (e != hipSuccess) {
-        *st = report_hip(e, "lu split leaf sync buffer");
+        *st = report_hip(e, "lu panel sync buffer");
         return nullptr;
     }
-    cache.push_back({dev, s, p});
-    return p;
+    cache.emplace_back(new PanelSync());
+    cache.back()->dev = dev;
+    cache.back()->stream = s;
+    cache.back()->ptr = p;
+    return cache.back().get();
 }
 
 template <typename T>
@@ -902,13 +910,14 @@ struct LuRec {
             ok(hipGetLastError(), "lu panel");
             return;
         }
-        uint64_t *sync = split_sync(s, &st);
+        PanelSync *sync = panel_sync(s, &st);
         if (!sync) return;
+        std::lock_guard<std::mutex> pair(sync->mu);
         hipLaunchKernelGGL((lu_panel_kernel<T, NB, R, NT, false>), dim3(g), dim3(NT), 0, s, (int)m, n, A, lda, ipiv,
-                           info, r0, sync, spin_limit);
+                           info, r0, sync->ptr, spin_limit);
         if (!ok(hipGetLastError(), "lu panel")) return;
         hipLaunchKernelGGL(lu_panel_recover_kernel<T>, dim3(1), dim3(PIV_THREADS), 0, s, m, n, A, lda, ipiv, info, r0,
-                           sync);
+                           sync->ptr);
         ok(hipGetLastError(), "lu panel recovery");
     }
 

@@ -9,6 +9,7 @@
 #pragma once
 
 #include <stdint.h>
+#include <stdlib.h>
 #include <string.h>
 #include <ucontext.h>
 
@@ -26,11 +27,19 @@
 #define __launch_bounds__(...)
 #define amdgpu_waves_per_eu(...)
 #define __align__(n) __attribute__((aligned(n)))
+#ifndef hipLaunchKernelGGL
 #define hipLaunchKernelGGL(...) ((void)0)
+#endif
 
 typedef void *hipStream_t;
-enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1 };
+#define hipStreamPerThread ((hipStream_t)2)
+enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorStreamCaptureUnsupported = 900 };
+enum hipStreamCaptureStatus { hipStreamCaptureStatusNone = 0, hipStreamCaptureStatusActive = 1 };
 inline hipError_t hipGetLastError() { return hipSuccess; }
+// for host code under test: what it allocates, and whether the stream is captured
+hipError_t hipGetDevice(int *dev);
+hipError_t hipMalloc(void **p, size_t bytes);
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *st);
 struct dim3 {
     unsigned x, y, z;
     dim3(unsigned x_ = 1, unsigned y_ = 1, unsigned z_ = 1) : x(x_), y(y_), z(z_) {}
@@ -159,6 +168,7 @@ inline bool run(int nt, int block, int grid, const std::vector<int> &order, std:
 }
 inline dim3 tid() { return dim3((unsigned)group()->cur, 0, 0); }
 inline int lane() { return group()->cur % 64; }
+inline int lane_of(int v, int l) { return meet(v).v[l]; }
 
 // D = A B + C in the lane layouts of the MFMA instructions, with fused steps in ascending k
 typedef double d4 __attribute__((ext_vector_type(4)));
@@ -206,6 +216,25 @@ inline int __all(int p) {
         if (!v.v[l]) return 0;
     return 1;
 }
+inline unsigned long long __ballot(int p) {
+    const auto v = emu::meet(p);
+    unsigned long long m = 0;
+    for (int l = 0; l < 64; ++l) m |= (unsigned long long)(v.v[l] != 0) << l;
+    return m;
+}
+inline int __ffsll(unsigned long long v) { return __builtin_ffsll((long long)v); }
+template <typename To, typename From>
+inline To emu_bits(From v) {
+    static_assert(sizeof(To) == sizeof(From), "the same bits");
+    To r;
+    memcpy(&r, &v, sizeof(To));
+    return r;
+}
+inline long long __double_as_longlong(double v) { return emu_bits<long long>(v); }
+inline double __longlong_as_double(long long v) { return emu_bits<double>(v); }
+inline unsigned __float_as_uint(float v) { return emu_bits<unsigned>(v); }
+inline float __uint_as_float(unsigned v) { return emu_bits<float>(v); }
+using std::fmax;
 template <typename T>
 inline T atomicExch(T *p, T v) {
     const T old = *p;
@@ -225,3 +254,11 @@ inline T atomicAdd(T *p, T v) {
 #define __builtin_amdgcn_wave_barrier() ((void)emu::meet(0))
 #define __builtin_amdgcn_sched_barrier(m) ((void)0)
 #define __builtin_amdgcn_s_setprio(p) ((void)0)
+#define __builtin_amdgcn_readlane(x, l) (emu::lane_of((int)(x), l))
+#define __builtin_amdgcn_readfirstlane(x) (emu::lane_of((int)(x), 0))
+// lane moves of DPP; not modelled
+#define __builtin_amdgcn_update_dpp(old, v, ctrl, rows, banks, bound) (abort(), (v))
+#define __HIP_MEMORY_SCOPE_AGENT 0
+#define __hip_atomic_store(p, v, order, scope) ((void)(*(p) = (v)))
+#define __hip_atomic_load(p, order, scope) (*(p))
+#define __hip_atomic_fetch_add(p, v, order, scope) (atomicAdd((p), (v)))

@@ -277,3 +277,45 @@ def test_interchanges_large(nla, m, n):
     err = L @ U - A0[:, cols][torch.from_numpy(p).to(DEV)]
     bound = 4 * n * 2.2e-16 * (L.abs() @ U.abs())
     assert torch.all(err.abs() <= bound)
+
+
+def test_threads_on_one_stream(nla, split_rows, spin_limit):
+    """Three host threads factor matrices of their own on one stream, with and
+    without waits that run out (a one-poll limit from the host): every thread's
+    factors are its own, as when it is alone."""
+    import threading
+    from nextla_amd import _lib
+    lib = _lib.load()
+    split_rows(1)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(9)
+    shapes = [(9000, 24), (700, 130), (3000, 64)]
+    A0 = [torch.empty((n, m), dtype=torch.float64, device=DEV).normal_(generator=g).t() for m, n in shapes]
+    ref = [nla.getrf2_(a.clone()) for a in A0]
+    stream = torch.cuda.Stream()
+    for limit in (0, 1):
+        spin_limit(limit)
+        work = [[a.clone() for _ in range(6)] for a in A0]
+        piv = [[torch.zeros(a.shape[1], dtype=torch.int64, device=DEV) for _ in range(6)] for a in A0]
+        info = [[torch.zeros(1, dtype=torch.int64, device=DEV) for _ in range(6)] for a in A0]
+        torch.cuda.synchronize()
+        bad = []
+
+        def run(i):
+            m, n = shapes[i]
+            for a, p, f in zip(work[i], piv[i], info[i]):
+                st = lib.nla_getrf2(_lib.NLA_F64, m, n, a.data_ptr(), m, p.data_ptr(), f.data_ptr(), stream.cuda_stream)
+                if st != 0:
+                    bad.append(st)
+        pool = [threading.Thread(target=run, args=(i,)) for i in range(3)]
+        for t in pool:
+            t.start()
+        for t in pool:
+            t.join()
+        torch.cuda.synchronize()
+        assert not bad
+        for i in range(3):
+            L, p, inf = ref[i]
+            for a, q, f in zip(work[i], piv[i], info[i]):
+                assert f.item() == inf == 0 and torch.equal(q, p)
+                assert torch.max(torch.abs(a - L)).item() <= 1e-12 * torch.max(torch.abs(L)).item()
