@@ -195,6 +195,107 @@ __global__ __launch_bounds__(PIV_THREADS) void lu_leaf_kernel(int64_t m, int n, 
     lu_leaf_body<T>(m, n, A, lda, ipiv, info, r0);
 }
 
+// The same leaf for up to REG_ROWS rows, held in registers from the first load
+// to the final store: one work-group, two barriers per column and nothing in
+// memory in between.  Its columns cost more with the rows (REG_RPT of them per
+// thread), those of the panel of several groups below do not, but that one has
+// a longer start and a recovery launch behind it: a call of few columns and
+// rows is faster here (narrow(), in LuRec).
+constexpr int REG_THREADS = 512, REG_RPT = 8, REG_ROWS = REG_THREADS * REG_RPT;
+
+template <typename T>
+__global__ __launch_bounds__(REG_THREADS) void lu_leaf_reg_kernel(int m, int n, T *__restrict__ A, int64_t lda,
+                                                                  int64_t *__restrict__ ipiv,
+                                                                  int64_t *__restrict__ info, int64_t r0) {
+    constexpr int W = REG_THREADS / 64;
+    __shared__ T s_val[W], s_sgn[W];
+    __shared__ int64_t s_row[W];
+    __shared__ T s_u[LEAF_COLS], s_o[LEAF_COLS];  // the pivot row, row j before the interchange
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int kmax = m < n ? m : n;
+    T a[REG_RPT][LEAF_COLS];
+#pragma unroll
+    for (int r = 0; r < REG_RPT; ++r) {
+        const int i = t + r * REG_THREADS;
+#pragma unroll
+        for (int c = 0; c < LEAF_COLS; ++c) a[r][c] = (i < m && c < n) ? A[i + (int64_t)c * lda] : T(0);
+    }
+#pragma unroll
+    for (int j = 0; j < LEAF_COLS; ++j) {
+        if (j >= kmax) break;
+        T bv = T(-1), bs = T(0);
+        int64_t bi = m;
+#pragma unroll
+        for (int r = 0; r < REG_RPT; ++r) {
+            const int i = t + r * REG_THREADS;
+            if (i >= j && i < m) better(bv, bs, bi, (T)fabs(a[r][j]), a[r][j], (int64_t)i);
+        }
+        wave_argmax(bv, bs, bi);
+        if (lane == 0) {
+            s_val[wv] = bv;
+            s_sgn[wv] = bs;
+            s_row[wv] = bi;
+        }
+        __syncthreads();
+        T pv = T(-1), av = T(0);
+        int64_t p = m;
+#pragma unroll
+        for (int w = 0; w < W; ++w) better(pv, av, p, s_val[w], s_sgn[w], s_row[w]);
+        const bool none = p >= m;  // no finite maximum (all NaN): keep row j
+        if (none) p = j;
+#pragma unroll
+        for (int r = 0; r < REG_RPT; ++r) {
+            const int i = t + r * REG_THREADS;
+            if (i == p) {
+#pragma unroll
+                for (int c = 0; c < LEAF_COLS; ++c) s_u[c] = a[r][c];
+            }
+            if (i == j) {
+#pragma unroll
+                for (int c = 0; c < LEAF_COLS; ++c) s_o[c] = a[r][c];
+            }
+        }
+        __syncthreads();
+        if (none) av = s_o[j];
+        if (t == 0) {
+            ipiv[j] = r0 + p + 1;
+            if (av == T(0) && *info == 0) *info = r0 + j + 1;
+        }
+        if (av != T(0)) {
+            const bool swap = p != j, recip = fabs(av) >= std::numeric_limits<T>::min();
+            const T rc = T(1) / av;
+#pragma unroll
+            for (int r = 0; r < REG_RPT; ++r) {
+                const int i = t + r * REG_THREADS;
+                if (swap && i == j) {
+#pragma unroll
+                    for (int c = 0; c < LEAF_COLS; ++c) a[r][c] = s_u[c];
+                } else if (swap && i == p) {
+#pragma unroll
+                    for (int c = 0; c < LEAF_COLS; ++c) a[r][c] = s_o[c];
+                }
+                if (i > j && i < m) {
+                    const T l = recip ? a[r][j] * rc : a[r][j] / av;
+                    a[r][j] = l;
+#pragma unroll
+                    for (int c = j + 1; c < LEAF_COLS; ++c) a[r][c] = a[r][c] - l * s_u[c];
+                }
+            }
+        }
+        // s_val is rewritten before the next column's first barrier, s_u after
+        // it: both were last read before one
+    }
+#pragma unroll
+    for (int r = 0; r < REG_RPT; ++r) {
+        const int i = t + r * REG_THREADS;
+        if (i < m) {
+#pragma unroll
+            for (int c = 0; c < LEAF_COLS; ++c)
+                if (c < n) A[i + (int64_t)c * lda] = a[r][c];
+        }
+    }
+}
+
 // The same factorization of a panel of up to NB columns, held in registers
 // by G work-groups of NT threads with R rows per thread from the first load
 // to the final store.  What bounds it is the chain of columns, not the
@@ -921,6 +1022,16 @@ struct LuRec {
         ok(hipGetLastError(), "lu panel recovery");
     }
 
+    // Few columns of more rows than a single group's panel takes (128): one
+    // group of the register leaf against a panel of several and its recovery
+    // launch.  Measured on MI355X (us per call, leaf / panel): FP64 256 x 1
+    // 6.2 / 10.3, 256 x 8 25.8 / 30.3, 1000 x 8 29.2 / 30.1, 2048 x 4
+    // 18.4 / 19.2, 2048 x 8 33.2 / 29.5, 4096 x 1 7.0 / 10.7, 4096 x 4
+    // 21.8 / 19.8; FP32 1000 x 8 25.7 / 27.9, 2048 x 8 28.9 / 26.9.
+    static bool narrow(int64_t m, int64_t n) {
+        return n <= LEAF_COLS && m > 128 && m <= REG_ROWS && m * n <= 12288;
+    }
+
     // an m x n panel, n <= panel_cols(m): 128-row groups up to 8192 rows (each
     // lane polls one group), 256 rows and more above
     void panel(int64_t m, int n, T *A, int64_t *ipiv, int64_t r0) {
@@ -965,6 +1076,12 @@ struct LuRec {
     void rec(int64_t m, int64_t n, T *A, int64_t *ipiv, int64_t r0) {
         if (st != NLA_OK || m == 0 || n == 0) return;
         const int nb = split_rows > 0 && m >= split_rows ? panel_cols(m) : 0;
+        if (nb > 0 && narrow(m, n)) {
+            hipLaunchKernelGGL(lu_leaf_reg_kernel<T>, dim3(1), dim3(REG_THREADS), 0, s, (int)m, (int)n, A, lda, ipiv,
+                               info, r0);
+            ok(hipGetLastError(), "lu register leaf");
+            return;
+        }
         if (n <= nb) {
             panel(m, (int)n, A, ipiv, r0);
             return;

@@ -319,3 +319,28 @@ def test_threads_on_one_stream(nla, split_rows, spin_limit):
             for a, q, f in zip(work[i], piv[i], info[i]):
                 assert f.item() == inf == 0 and torch.equal(q, p)
                 assert torch.max(torch.abs(a - L)).item() <= 1e-12 * torch.max(torch.abs(L)).item()
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("m,n", [(128, 8), (129, 8), (1024, 8), (1536, 8), (1537, 8), (2048, 5), (4096, 3), (4096, 1),
+                                 (4097, 1), (513, 2)])
+def test_narrow_blocks(nla, split_rows, dtype, m, n):
+    """Few columns, at the edges of the rule between the single group's panel,
+    the register leaf and the panel of several groups: the pivots and factors
+    of the global-memory leaf, with a tied first column, a zero column and a
+    column of NaN among the inputs."""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + n)
+    for kind in ("ties", "zero", "nan"):
+        A0 = torch.empty((n, m), dtype=dtype, device=DEV).normal_(generator=g).t()
+        A0[:, n // 2] = {"ties": 1.0, "zero": 0.0, "nan": float("nan")}[kind]
+        split_rows(0)
+        L1, p1, i1 = nla.getrf2_(A0.clone())
+        split_rows(1)
+        L2, p2, i2 = nla.getrf2_(A0.clone())
+        assert i1 == i2 == (n // 2 + 1 if kind == "zero" else 0), kind
+        assert torch.equal(p1, p2), kind
+        assert torch.equal(torch.isnan(L1), torch.isnan(L2)), kind
+        tol = 1e-12 if dtype == torch.float64 else 1e-5
+        L1, L2 = torch.nan_to_num(L1), torch.nan_to_num(L2)
+        assert torch.max(torch.abs(L1 - L2)).item() <= tol * torch.max(torch.abs(L1)).item(), kind
