@@ -568,8 +568,9 @@ int32_t nla_serve_destroy(nla_server server);
  *                      trans 'T', right side with 'N');
  *                      above 512 rows FP64 panels use 16 columns per group;
  *   NLA_CFG_PANEL_STRIP_F32 / _F64: right-hand-side columns per panel
- *                      work-group, 16 (default; eight-wave panels take
- *                      32 where there are more than 4096) or 32;
+ *                      work-group, 16 (default: at least that; above
+ *                      4096 columns eight-wave panels take 32 where that is
+ *                      faster) or 32;
  *   NLA_CFG_PANEL_WAVES: waves per panel work-group (panels up to 512 rows):
  *                      4 (left-looking, 16 columns, two and more groups per
  *                      CU) or 8 (32-row units, right-looking TRSM); 0

@@ -500,8 +500,8 @@ __global__ __launch_bounds__(256) void panel_left_kernel(int nbig, int64_t m, co
 //     used.  The loops have no load under a branch (the compiler would wait
 //     at the join): a wave's steps are split by which of its units are still
 //     active, and the waves that apply the inverse run their own copy;
-//   - TRMM has no chain: every wave forms units w and 15 - w, whose parts of
-//     the triangle add up to the same, from the strip in LDS.
+//   - TRMM has no chain: the waves form whole units from the strip in LDS, long
+//     ones paired with short ones.
 
 template <typename T>
 struct Mat2 {
@@ -929,9 +929,11 @@ __device__ __forceinline__ void panel_trmm(int nbig, int64_t m, int64_t c0, cons
     const int nu = (nbig + 31) / 32;
     const NLA_LDS T *xb = bs + lo * LDB + kk;
     for (int j = 0; j < 2; ++j) {
-        // units w and 2 nw - 1 - w of the nu: parts of the triangle that add up alike
-        const int u = j == 0 ? wv : 2 * PU_WAVES - 1 - wv;
-        if (u >= nu) continue;
+        // a unit each for the longest ones, and the shortest for the waves with
+        // the shortest of those: by length, units nu - 1 - w and nu - 16 + w,
+        // from the panel's top down (512 rows, 64 columns: 5 % slower upwards)
+        const int q = (j == 1) == lower ? nu - 1 - wv : nu - 2 * PU_WAVES + wv, u = lower ? q : nu - 1 - q;
+        if (q < 0) continue;
         const int r0 = 32 * u;
         PanelAcc<T, 2, CBW> acc;
         acc.zero();
@@ -1113,34 +1115,60 @@ static hipError_t launch_panel_left_n(const PanelArgs<T> &a, hipStream_t s) {
     return launch_panel_left<T, 1024, TRMM>(a, s);
 }
 
+// Right-hand sides per group of the eight-wave panel, or 0 for the
+// left-looking strip (16 of them).  kc: M contiguous along k; bcol: B's
+// contiguous direction runs along the right-hand sides; n x n panel, m of them.
+//
+// An eight-wave group has a CU to itself.  32 columns halve the reads of M and
+// fill the matrix cores better, but a round of such groups is 8192 columns, so
+// they win where they leave less than half of the last round idle (full).  Four
+// waves and 16 columns leave room for two and more groups on a CU: the
+// left-looking strip wins where there is little of a chain to shorten, or, for
+// TRSM, more strips than CUs to hide it, but it loads M along k (kc) one
+// element per cache line.  It also rounds more (TRSM of an upper M twice as
+// much, TRMM above 192 rows 1.2 to 1.6 times), so of two that take about as
+// long the eight waves are taken.  Within 1 % of the fastest of the three on
+// average over 64 .. 512 rows and 16 .. 24000 columns.  Measured on MI355X (us,
+// left / eight waves of 16 / of 32 columns, TRSM with its inverses):
+//   FP64 TRSM  L-L-T 128 rows, 10000 columns 29.0 / 37.8 / 73.9; 144 rows 38.5 / 48.6 / 84.7;
+//              512 rows, 8192 131 / 105 / 110; R-U-N 149 / 120 / 113; L-L-N 81.6 / 86.0 / 103
+//   FP64 TRMM  L-L-N 128 rows, 10000 16.8 / 20.2 / 34.8; 320 rows 50.1 / 42.0 / 60.0;
+//              L-L-T 256 rows, 8192 42.5 / 32.7 / 25.4; 10000 57.7 / 43.2 / 43.5
+//   FP32 TRSM  L-L-T 512 rows, 8192 119 / 62.4 / 54.5; 10000 167 / 81.6 / 91.5; R-U-N 211 / 122 / 99.9
+//   FP32 TRMM  L-L-N 144 rows, 10000 18.3 / 13.5 / 24.5; R-U-N 512 rows, 8192 126 / 50.2 / 37.9
+// (32 columns for all past 4096: up to 1.9 times as long as what it replaced).
+template <typename T>
+static int panel_columns(bool trmm, bool kc, bool bcol, bool unit, int n, int64_t m) {
+    constexpr bool F64 = sizeof(T) == 8;
+    // few columns.  A unit diagonal is LU's: its blocks are as often flagged
+    // for refinement as not, which the eight waves do on MFMA (64 rows 25 / 8
+    // us, 128 rows 48 / 15)
+    if (m <= 16 * 256) return n > 128 || (trmm ? !(F64 && kc && bcol) : unit) ? 16 : 0;
+    const bool full = (m - 1) % (32 * 256) >= 16 * 256;
+    if (n <= 64) return 0;
+    if (!trmm) {
+        if (!F64 && bcol && full) return 32;
+        if (!kc || n <= 128) return 0;
+        if (F64) return bcol && n > 384 && full ? 32 : 16;
+        return bcol || (n > 256 && full) ? 32 : 16;
+    }
+    if (F64) {
+        if (n <= 128 || (!kc && n <= 192 && m > 32 * 256)) return 0;
+        return full || (kc && n > 384) ? 32 : 16;
+    }
+    if (bcol) return full ? 32 : (!kc && n <= 128 ? 0 : 16);
+    return n > 320 && full ? 32 : 16;
+}
+
 template <typename T>
 hipError_t launch_panel(const PanelArgs<T> &a, hipStream_t s) {
     if (a.m <= 0 || a.nbig <= 0) return hipSuccess;
     if (a.nbig > PANEL_MAX) return hipErrorInvalidValue;
     if (a.strip != 16 && a.strip != 32) return hipErrorInvalidValue;
-    // Four waves and 16 columns leave room for two and more work-groups on a
-    // CU: the left-looking strip wins where a TRSM has more strips than CUs and
-    // M's columns are contiguous (along k it loads one element per cache line),
-    // or where there is no chain to shorten.  Otherwise, more strips
-    // than CUs take 32 columns a group, which halves the reads of M.  Measured on MI355X (us, left / eight waves): FP64
-    // TRSM of 512 rows with 64 / 4096 / 8192 columns 40.2 / 32.8, 47.9 / 41.0,
-    // 75.0 / 80.8, 128 rows 7.0 / 7.5, 64 rows 4.4 / 4.5; FP64 TRMM 512 rows
-    // 37.8 / 23.8, 45.5 / 30.8, 72.6 / 59.8, 128 rows 6.7 / 5.8 and with 8192
-    // columns 11.2 / 12.2; FP32 TRSM 512 rows 27.6 / 22.9, 30.9 / 26.1,
-    // 46.6 / 49.7, TRMM 27.1 / 17.9, 30.1 / 22.3, 47.7 / 43.8.  Whole calls of
-    // n = 2048 with 8192 columns (left / eight waves of 16 / of 32 columns):
-    // FP64 TRSM L-L-N 748 / 770 / 805, L-L-T 961 / 860 / 833, FP32 L-L-N
-    // 434 / 450 / 435, L-L-T 685 / 446 / 423; FP64 TRMM L-L-N 719 / 669 / 646,
-    // L-L-T 977 / 777 / 663, FP32 421 / 406 / 394, 720 / 396 / 371; with 3000
-    // columns 16 win throughout (FP64 L-L-T 484 / 645, TRMM 446 / 492).
-    // A unit diagonal is LU's: its blocks are as often flagged for refinement
-    // as not, which the eight waves do on MFMA (in the LU of n = 8192, left-looking /
-    // eight waves: 64 rows 25 / 8 us, 128 rows 48 / 15).
-    const bool many = a.m > 16 * 256, small = a.nbig <= 128 && !a.unit, left = a.trmm ? many && small
-                                                                                      : (many && a.mrs == 1) || small;
-    if (a.nbig > PU_MAX || a.waves == 4 || (a.waves == 0 && a.strip != 32 && left))
+    const int columns = a.strip == 32 ? 32 : panel_columns<T>(a.trmm, a.mcs == 1, a.brs != 1, a.unit, a.nbig, a.m);
+    if (a.nbig > PU_MAX || a.waves == 4 || (a.waves == 0 && columns == 0))
         return a.trmm ? launch_panel_left_n<T, true>(a, s) : launch_panel_left_n<T, false>(a, s);
-    return a.strip == 32 || many ? launch_panel_w<T, 32>(a, s) : launch_panel_w<T, 16>(a, s);
+    return columns == 32 ? launch_panel_w<T, 32>(a, s) : launch_panel_w<T, 16>(a, s);
 }
 
 template hipError_t launch_panel<float>(const PanelArgs<float> &, hipStream_t);

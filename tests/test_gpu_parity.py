@@ -399,3 +399,39 @@ def test_panels_many_columns(nla, dt, n, m):
         Ad, Bd = (torch.from_numpy(np.ascontiguousarray(t.T)).cuda().t() for t in (A, B))
         nla.unified_rectrxm_(side, uplo, trans, 1.5, func, Ad, Bd)
         check_bound(side, uplo, trans, 1.5, func, A, B, Bd.cpu().numpy())
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n,m", [(64, 4097), (65, 4097), (128, 8192), (129, 8193), (160, 8193), (192, 8192),
+                                 (193, 8200), (256, 4097), (257, 12288), (320, 12289), (321, 8192), (384, 8193),
+                                 (385, 8193), (512, 8192), (512, 12289)])
+def test_panel_rule_edges(nla, dt, n, m):
+    """The panels at the edges of the rule between the left-looking strip and
+    eight waves with 16 or 32 columns a group, every side / uplo / trans, TRSM
+    and TRMM, unit and general diagonals, in float64 on the device: the product
+    elementwise within (n + 3) eps |op(A)||B| (n + 1 roundings of a sum in any
+    order, one of the scale), the solution's residual within 10 n eps
+    |op(A)||X| (substitution in 64-blocks: the bound of the tests above)."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + m)
+    eps_ = torch.finfo(dt).eps
+    T = torch.empty((n, n), dtype=dt, device="cuda").uniform_(-1, 1, generator=g).tril_(-1) / n ** 0.5
+    T.diagonal().uniform_(2, 3, generator=g)
+    for (side, uplo, trans, func), diag in itertools.product(itertools.product("LR", "LU", "NT", "SM"), "NU"):
+        A = (T if uplo == "L" else T.t()).t().contiguous().t()
+        shape = (m, n) if side == "L" else (n, m)
+        B = torch.empty(shape, dtype=dt, device="cuda").normal_(generator=g).t()
+        op = A.double().clone()
+        if diag == "U":
+            op.diagonal().fill_(1.0)
+        op = op if trans == "N" else op.t()
+        X = B.clone()
+        (nla.trsm if func == "S" else nla.trmm)(side, uplo, trans, diag, A, X, 1.5)
+        prod = (lambda t: op @ t) if side == "L" else (lambda t: t @ op)
+        absp = (lambda t: op.abs() @ t.abs()) if side == "L" else (lambda t: t.abs() @ op.abs())
+        Bd, Xd = B.double(), X.double()
+        if func == "M":
+            err, bound = (Xd - 1.5 * prod(Bd)).abs(), 1.5 * (n + 3) * eps_ * absp(Bd)
+        else:
+            err, bound = (prod(Xd) - 1.5 * Bd).abs(), 10 * n * eps_ * absp(Xd)
+        assert torch.all(err <= bound), (side, uplo, trans, func, diag, (err / bound).max().item())
