@@ -170,6 +170,40 @@ static hipError_t launch_tri_dense(const GemmArgs<T> &a, hipStream_t s) {
     }
 }
 
+// Tile shape by the time its rounds take: ceil(tiles / CUs) rounds of the
+// tile's area at the rate its shape reaches with full rounds, for K and
+// the depth k0 that a round's start and end are worth.  Rates measured on
+// MI355X (TFLOP/s): FP64 256 x 128 67, 128 x 128 62, 64 x 128 50; FP32
+// 256 x 256 137 (one group per CU, so nothing hides its start and end),
+// 128 x 128 131 (114 with ragged edges or one group per CU), 64 x 64 126.
+// E.g. FP64 3000^3 1515 / 1230 / 1353 us, 6000 x 1024 x 1024
+// 269 / 289 / 317; FP32 6000 x 2048 x 2048 550 / 446 / 415,
+// 1024 x 8192 x 1024 256 / 140 / 144, 512 x 8192 x 512 - / 47 / 42,
+// 3333 x 4444 x 555 186 / 170 / 162.
+template <typename T>
+int gemm_tile_shape(int64_t M, int64_t N, int64_t K, double *us) {
+    auto cost = [&](int bm, int bn, double rate, int k0) {
+        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        return (double)((tiles + 255) / 256) * bm * bn / rate * (double)(K + k0);
+    };
+    double c[3];
+    if constexpr (sizeof(T) == 8) {
+        c[0] = cost(256, 128, 67, 0);
+        c[1] = cost(128, 128, 62, 0);
+        c[2] = cost(64, 128, 50, 0);
+    } else {
+        const bool slow = M % 128 != 0 || N % 128 != 0 || (M / 128) * (N / 128) <= 256;
+        c[0] = cost(256, 256, 137, 100);
+        c[1] = cost(128, 128, slow ? 114 : 131, 30);
+        c[2] = cost(64, 64, 126, 30);
+    }
+    const int shape = c[0] <= c[1] && c[0] <= c[2] ? 0 : (c[1] <= c[2] ? 1 : 2);
+    if (us != nullptr) *us = c[shape] * (2 * 256 * 1e-6);  // 2 flops on each of 256 CUs, TFLOP/s
+    return shape;
+}
+template int gemm_tile_shape<float>(int64_t, int64_t, int64_t, double *);
+template int gemm_tile_shape<double>(int64_t, int64_t, int64_t, double *);
+
 template <typename T>
 hipError_t launch_gemm_tiled(const GemmArgs<T> &a, hipStream_t s) {
     if (a.M <= 0 || a.N <= 0) return hipSuccess;
@@ -186,32 +220,15 @@ hipError_t launch_gemm_tiled(const GemmArgs<T> &a, hipStream_t s) {
         if constexpr (sizeof(T) == 8) return launch_tri<T, 32, 64, 32, 2, 2>(a, s);
         else return launch_tri<T, 64, 64, 32, 2, 2>(a, s);
     }
-    // Tile shape by the time its rounds take: ceil(tiles / CUs) rounds of the
-    // tile's area at the rate its shape reaches with full rounds, for K and
-    // the depth k0 that a round's start and end are worth.  Rates measured on
-    // MI355X (TFLOP/s): FP64 256 x 128 67, 128 x 128 62, 64 x 128 50; FP32
-    // 256 x 256 137 (one group per CU, so nothing hides its start and end),
-    // 128 x 128 131 (114 with ragged edges or one group per CU), 64 x 64 126.
-    // E.g. FP64 3000^3 1515 / 1230 / 1353 us, 6000 x 1024 x 1024
-    // 269 / 289 / 317; FP32 6000 x 2048 x 2048 550 / 446 / 415,
-    // 1024 x 8192 x 1024 256 / 140 / 144, 512 x 8192 x 512 - / 47 / 42,
-    // 3333 x 4444 x 555 186 / 170 / 162.
-    auto cost = [&](int bm, int bn, double rate, int k0) {
-        const int64_t tiles = ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
-        return (double)((tiles + 255) / 256) * bm * bn / rate * (double)(a.K + k0);
-    };
+    const int shape = gemm_tile_shape<T>(a.M, a.N, a.K, nullptr);
     if constexpr (sizeof(T) == 8) {
-        const double c1 = cost(256, 128, 67, 0), c2 = cost(128, 128, 62, 0), c3 = cost(64, 128, 50, 0);
-        if (c1 <= c2 && c1 <= c3) return launch_tri_dense<T, 256, 128, 16, 4, 2>(a, s);
-        if (c2 <= c3) return launch_tri_dense<T, 128, 128, 16, 4, 2>(a, s);
+        if (shape == 0) return launch_tri_dense<T, 256, 128, 16, 4, 2>(a, s);
+        if (shape == 1) return launch_tri_dense<T, 128, 128, 16, 4, 2>(a, s);
         return launch_tri_dense<T, 64, 128, 16, 2, 2>(a, s);
     } else {
         if (a.tri) return hipErrorInvalidValue;  // triangular products are FP64 only
-        const bool slow = a.M % 128 != 0 || a.N % 128 != 0 || (a.M / 128) * (a.N / 128) <= 256;
-        const double c1 = cost(256, 256, 137, 100), c2 = cost(128, 128, slow ? 114 : 131, 30),
-                     c3 = cost(64, 64, 126, 30);
-        if (c1 <= c2 && c1 <= c3) return launch_trans<T, 256, 256, 32, 4, 4, 0>(a, s);
-        if (c2 <= c3) return launch_trans<T, 128, 128, 32, 2, 2, 0>(a, s);
+        if (shape == 0) return launch_trans<T, 256, 256, 32, 4, 4, 0>(a, s);
+        if (shape == 1) return launch_trans<T, 128, 128, 32, 2, 2, 0>(a, s);
         return launch_trans<T, 64, 64, 32, 2, 2, 0>(a, s);
     }
 }

@@ -57,22 +57,26 @@ hipError_t launch_split(const GemmArgs<T> &a, hipStream_t s) {
 template <typename T>
 hipError_t launch_gemm(const GemmArgs<T> &a, hipStream_t s) {
     if (a.M <= 0 || a.N <= 0) return hipSuccess;
-    // Measured on MI355X (us per launch, tiled / split): FP64 512^3 (K = 256)
-    // 28.7 / 7.1, 1024 x 1024 x 1024 103 / 47, 64 x 4096 x 4096 390 / 40,
-    // 4096 x 8 x 4096 523 / 38, 3000 x 1000 x 512 105 / 69, 1792 x 1792 x 256
-    // 47 / 48, 2048 x 2048 x 256 45 / 60, and with K = 64, where C's traffic
-    // counts, 1024 x 1024 11.8 / 11.6, 1280 x 1280 12.4 / 15.2.  FP32, whose
-    // smallest tile is 64 x 64: 512 x 512 x 256 9.2 / 5.4, 768 x 768 x 1024
-    // 26.8 / 21.7, 1024 x 1024 x 256 10.2 / 11.8, 64 x 4096 x 4096 97 / 31,
-    // 256 x 4096 x 4096 101 / 100.  Eight waves per tile, 64 x 16 and 64 x 64
-    // tiles were within 10 % of 32 x 32 with four or slower.  FP64 with op(X)
-    // transposed, whose lanes load from 16 rows of memory, reaches 36 TFLOP/s
-    // here (48 otherwise): a block reflector of 8192 x 8192 with k = 256, 128
-    // tiles, takes 1453 / 1700 us tiled / split.
+    // Split where its estimated time is the shorter: q tiles of 32 x 32 per CU,
+    // each with a start and end of 0.6 us and the rate of its orientation (with
+    // op(X) transposed a lane loads from 16 rows of memory), against the rounds
+    // of the tiled kernels and the 1.6 us that their first and last steps take
+    // more.  Within 0.5 % of the faster one on average over K = 16 .. 4096 and
+    // 16 to 4096 tiles of 32 x 32, at most 10 % slower where the tiles are
+    // square and fill the last round.  Measured on MI355X (us per launch, tiled /
+    // split): FP64 64 x 4096 x 4096 371 / 50, 1024^3 89 / 48, 1536 x 1536 x 192
+    // 32.5 / 33.5, 1408 x 1408 x 192 22.9 / 30.2, 1024 x 1024 x 48 9.5 / 10.0,
+    // with X transposed 9.3 / 12.2, 1152 x 1152 x 192 so 21.4 / 30.5; FP32
+    // 512 x 512 x 192 6.6 / 4.8, 768 x 768 x 64 4.8 / 5.5, 768 x 768 x 1024
+    // 24 / 23, 256 x 4096 x 4096 97 / 118.
     if (a.leaf == 0 && a.tri == 0 && a.K > 0) {
-        auto tiles = [&](int b) { return ((a.M + b - 1) / b) * ((a.N + b - 1) / b); };
-        const bool split = sizeof(T) == 8 ? tiles(128) <= (a.K < 128 ? 64 : (a.tx ? 96 : 192)) : tiles(64) <= 144;
-        if (split) return launch_split<T, 2, 2, 4>(a, s);
+        constexpr bool F64 = sizeof(T) == 8;
+        const int64_t tiles = ((a.M + 31) / 32) * ((a.N + 31) / 32), q = (tiles + 255) / 256;
+        const double rate = F64 ? (a.tx ? (a.ty ? 0.0104 : 0.0150) : (a.ty ? 0.0090 : 0.0094))
+                                : (a.tx ? (a.ty ? 0.0070 : 0.0074) : 0.0062);  // us per k and tile of a CU
+        double tiled = 0;
+        gemm_tile_shape<T>(a.M, a.N, (a.K + 15) / 16 * 16, &tiled);
+        if ((double)q * (0.6 + rate * (double)(a.K + (F64 ? 16 : 32))) < tiled + 1.6) return launch_split<T, 2, 2, 4>(a, s);
     }
     return launch_gemm_tiled<T>(a, s);
 }

@@ -200,6 +200,10 @@ template <typename T>
 hipError_t launch_gemm(const GemmArgs<T> &a, hipStream_t s);
 template <typename T>
 hipError_t launch_gemm_tiled(const GemmArgs<T> &a, hipStream_t s);
+// Tile shape of a tiled product (0: the largest), and its estimated kernel time
+// in us (us nullable).
+template <typename T>
+int gemm_tile_shape(int64_t M, int64_t N, int64_t K, double *us);
 
 template <typename T>
 hipError_t launch_leaf(const LeafArgs<T> &a, hipStream_t s);

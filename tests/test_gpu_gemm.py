@@ -43,3 +43,27 @@ def test_every_orientation(nla, dtype, m, n, k):
                                   torch.cuda.current_stream().cuda_stream)
                 assert st == 0
                 assert torch.all((C.double() - 1.5 * P).abs() <= 1.5 * (k + 3) * eps * A), (xt, yt, pad, "beta 0")
+
+
+def check(nla, dtype, m, n, k, pads):
+    """C -= X*Y in every orientation, within (k + 3) eps (|C| + |X||Y|)."""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + 7 * n + 31 * k)
+    eps = torch.finfo(dtype).eps
+    for xt in (False, True):
+        for yt in (False, True):
+            for pad in pads:
+                X, Y, C = mat(m, k, dtype, xt, pad, g), mat(k, n, dtype, yt, pad, g), mat(m, n, dtype, False, pad, g)
+                Xd, Yd, Cd = X.double(), Y.double(), C.double()
+                ref, bound = Cd - Xd @ Yd, (k + 3) * eps * (Cd.abs() + Xd.abs() @ Yd.abs())
+                nla.GEMM_SUB_(C, X, Y)
+                assert torch.all((C.double() - ref).abs() <= bound), (xt, yt, pad)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(20001, 24, 100), (24, 20001, 100), (597, 864, 8), (768, 769, 1024), (1408, 1408, 192),
+                                   (1152, 1152, 192), (1024, 1024, 48)])
+def test_between_the_kernels(nla, dtype, m, n, k):
+    """Shapes near the line between the K-splitting and the tiled kernels,
+    long and narrow ones among them."""
+    check(nla, dtype, m, n, k, (0, 3))
