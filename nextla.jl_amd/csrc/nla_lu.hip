@@ -9,8 +9,8 @@
 // A22 -= A21 A12, factor A22 and apply its interchanges to the left block.
 // Panels of up to 64 columns are one kernel (the same eliminations with
 // rank-1 updates in place of the GEMMs of that width), held in registers by
-// up to 128 work-groups that exchange one pivot row per column (32 columns
-// above 32,768 rows, 16 above 65,536; past 131,072 rows 8 columns in global
+// up to 128 work-groups that exchange one pivot row per column (fewer columns
+// from 16,384 rows on, in FP32 32,768; past 131,072 rows 8 columns in global
 // memory).  Pivots are kept as global rows throughout (the reference shifts
 // them by n1 after each recursive call).  Everything is enqueued on the
 // caller's stream; pivots and info stay on the device.
@@ -328,18 +328,23 @@ __global__ __launch_bounds__(REG_THREADS) void lu_leaf_reg_kernel(int m, int n, 
 // launches between them.  Groups of 64, 128 and 256 rows measure alike; all
 // groups on one XCD, with agent- or L2-scope words, is no faster.
 //
-// At most LU_MAX_WG groups are launched, which an idle part of the chip
-// holds at once; a cooperative launch would guarantee it, but costs about
-// 150 us once other streams have been used.  Each wait is bounded, so a
-// group that is not resident (another persistent grid holds the CUs) cannot
-// hang the others.  Every group saves its rows before its first exchange
-// (and group 0 the prior info), and a wait that runs out raises a flag; the
-// one-work-group recovery launch that follows every such panel returns at
-// once unless the flag is up, and otherwise restores the saved block and
-// factors it with the global-memory leaf, so the factorization stays exact.
+// The groups of a panel wait for each other, so they must all get a place.  At
+// most LU_MAX_WG are launched, on at most 64 CUs (LU_CUS: the rows of one group
+// times its columns fill half of a CU's LDS, or a whole one's with 64 groups):
+// a process runs four kernels at a time unless it asks for more hardware
+// queues, so four LUs on streams of their own, of any height, hold the chip
+// together instead of keeping parts of it from each other.  A cooperative
+// launch would guarantee a place, but costs about 150 us once other streams
+// have been used.  Each wait is bounded, so a group that is not resident
+// (another persistent grid holds the CUs) cannot hang the others.  Every group
+// saves its rows before its first exchange (and group 0 the prior info), and a
+// wait that runs out raises a flag; the one-work-group recovery launch that
+// follows every such panel returns at once unless the flag is up, and
+// otherwise restores the saved block and factors it with the global-memory
+// leaf, so the factorization stays exact.
 // A single group (ONE) exchanges nothing: one barrier per column.
 constexpr int LU_MAX_WG = 128;              // groups of one panel (two polled per lane)
-constexpr int LU_WORDS = 64;                // registers of a row: NB * R
+constexpr int LU_CUS = 64;                  // compute units that a panel may hold: a quarter of the chip
 constexpr int SYNC_EPOCH = 0, SYNC_LEAVE = 1;
 // words 2, 3 of the buffer: the timeout flag and the info value saved before
 // the panel; then, for both parities, the groups' candidates (three arrays of
@@ -349,8 +354,12 @@ constexpr int SYNC_FLAG = 2, SYNC_INFO = 3;
 constexpr int SYNC_SLOTS = 64, HEAD_WORDS = 3 * LU_MAX_WG, ROW_WORDS = 136;
 constexpr int PAR_WORDS = HEAD_WORDS + LU_MAX_WG * ROW_WORDS;
 constexpr int SYNC_WORDS = SYNC_SLOTS + 2 * PAR_WORDS;
-constexpr int64_t PANEL_M_MAX = 256 * LU_MAX_WG;  // rows of a 64-column panel
-constexpr int64_t SYNC_BYTES = SYNC_WORDS * 8 + PANEL_M_MAX * LU_WORDS * 8;
+// rows of a 64-column panel: half the columns for twice as many, and so on
+template <typename T>
+constexpr int64_t PANEL_M_MAX = sizeof(T) == 8 ? 64 * 256 : 128 * 256;
+constexpr int64_t PANEL_M_ALL = 131072;  // rows of any panel
+constexpr int64_t SYNC_BYTES = SYNC_WORDS * 8 + PANEL_M_MAX<double> * 64 * 8;
+static_assert(PANEL_M_MAX<double> * 8 == PANEL_M_MAX<float> * 4, "one buffer serves both types");
 constexpr int64_t SPLIT_SPIN_LIMIT = int64_t(1) << 20;  // about a second of polling
 
 __device__ inline void st_agent(uint64_t *p, uint64_t v) {
@@ -360,10 +369,12 @@ __device__ inline uint64_t ld_agent(const uint64_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Columns of the register panel for m rows (a row's NB * R registers are the
-// same for every height), 0 where the panel does not take them.
+// Columns of the register panel for m rows, 0 where the panel does not take them.
+template <typename T>
 inline int panel_cols(int64_t m) {
-    return m <= PANEL_M_MAX ? 64 : (m <= 2 * PANEL_M_MAX ? 32 : (m <= 4 * PANEL_M_MAX ? 16 : 0));
+    int nb = 64;
+    for (int64_t most = PANEL_M_MAX<T>; m > most && nb > 8; most *= 2) nb /= 2;
+    return m <= PANEL_M_ALL ? nb : 0;
 }
 
 __device__ __forceinline__ double lane_double(double v, int l) {
@@ -413,7 +424,7 @@ __global__ __launch_bounds__(NT) void lu_panel_kernel(int m, int n, T *__restric
                                                       int64_t *__restrict__ ipiv, int64_t *__restrict__ info,
                                                       int64_t r0, uint64_t *__restrict__ sync, int64_t spin_limit) {
     constexpr int W = NT / 64, ROWS = NT * R;
-    static_assert(NB <= 64 && NB % 16 == 0, "a wave publishes one row");
+    static_assert(NB == 8 || (NB <= 64 && NB % 16 == 0), "a wave publishes one row");
     __shared__ T s_l[NB][ROWS];                                       // finished columns (and rows of U)
     __shared__ __attribute__((aligned(16))) T s_row[2][W][NB + 2];    // each wave's candidate row, entry c at c + 1
     __shared__ __attribute__((aligned(16))) T s_u[2][NB + 2];         // the pivot row, entry c at c + 1; 1 / pivot at 0
@@ -720,7 +731,7 @@ __global__ __launch_bounds__(NT) void lu_panel_kernel(int m, int n, T *__restric
     }
     if constexpr (NB >= 32)
         for (; good && j < kmax && j < NB - 16; ++j) run(j, std::integral_constant<int, 32>{});
-    for (; good && j < kmax; ++j) run(j, std::integral_constant<int, 16>{});
+    for (; good && j < kmax; ++j) run(j, std::integral_constant<int, NB < 16 ? NB : 16>{});
     __syncthreads();
     // a row's entries are in its own thread's column of LDS (rows of U were
     // written there by another wave, before the barrier)
@@ -1002,8 +1013,11 @@ struct LuRec {
     int64_t split_rows = lu_split_rows();
     int64_t spin_limit = lu_spin_limit() > 0 ? lu_spin_limit() : SPLIT_SPIN_LIMIT;
 
-    template <int NB, int R, int NT>
+    // the register panel for up to MOST rows
+    template <int NB, int R, int NT, int MOST>
     void panel_of(int64_t m, int n, T *A, int64_t *ipiv, int64_t r0) {
+        constexpr int GROUPS = MOST / (NT * R), PER_CU = 163840 / (NB * NT * R * (int)sizeof(T) + 6144);
+        static_assert(GROUPS <= LU_MAX_WG && GROUPS <= LU_CUS * PER_CU, "every group gets a place");
         const unsigned g = (unsigned)((m + NT * R - 1) / (NT * R));
         if (g == 1) {
             hipLaunchKernelGGL((lu_panel_kernel<T, NB, R, NT, true>), dim3(1), dim3(NT), 0, s, (int)m, n, A, lda, ipiv,
@@ -1035,11 +1049,19 @@ struct LuRec {
     // an m x n panel, n <= panel_cols(m): 128-row groups up to 8192 rows (each
     // lane polls one group), 256 rows and more above
     void panel(int64_t m, int n, T *A, int64_t *ipiv, int64_t r0) {
-        const int nb = panel_cols(m);
-        if (nb == 64 && m <= 8192) panel_of<64, 1, 128>(m, n, A, ipiv, r0);
-        else if (nb == 64) panel_of<64, 1, 256>(m, n, A, ipiv, r0);
-        else if (nb == 32) panel_of<32, 2, 256>(m, n, A, ipiv, r0);
-        else panel_of<16, 4, 256>(m, n, A, ipiv, r0);
+        const int nb = panel_cols<T>(m);
+        if constexpr (sizeof(T) == 8) {
+            if (nb == 64 && m <= 8192) panel_of<64, 1, 128, 8192>(m, n, A, ipiv, r0);
+            else if (nb == 64) panel_of<64, 1, 256, 16384>(m, n, A, ipiv, r0);
+            else if (nb == 32) panel_of<32, 1, 256, 32768>(m, n, A, ipiv, r0);
+            else if (nb == 16) panel_of<16, 2, 256, 65536>(m, n, A, ipiv, r0);
+            else panel_of<8, 4, 256, 131072>(m, n, A, ipiv, r0);
+        } else {
+            if (nb == 64 && m <= 8192) panel_of<64, 1, 128, 8192>(m, n, A, ipiv, r0);
+            else if (nb == 64) panel_of<64, 1, 256, 32768>(m, n, A, ipiv, r0);
+            else if (nb == 32) panel_of<32, 2, 256, 65536>(m, n, A, ipiv, r0);
+            else panel_of<16, 4, 256, 131072>(m, n, A, ipiv, r0);
+        }
     }
 
     bool ok(hipError_t e, const char *where) {
@@ -1075,7 +1097,7 @@ struct LuRec {
     // reference's "ipiv[i] += n1" (src/lu.jl:289-291) makes of them.
     void rec(int64_t m, int64_t n, T *A, int64_t *ipiv, int64_t r0) {
         if (st != NLA_OK || m == 0 || n == 0) return;
-        const int nb = split_rows > 0 && m >= split_rows ? panel_cols(m) : 0;
+        const int nb = split_rows > 0 && m >= split_rows ? panel_cols<T>(m) : 0;
         if (nb > 0 && narrow(m, n)) {
             hipLaunchKernelGGL(lu_leaf_reg_kernel<T>, dim3(1), dim3(REG_THREADS), 0, s, (int)m, (int)n, A, lda, ipiv,
                                info, r0);

@@ -344,3 +344,54 @@ def test_narrow_blocks(nla, split_rows, dtype, m, n):
         tol = 1e-12 if dtype == torch.float64 else 1e-5
         L1, L2 = torch.nan_to_num(L1), torch.nan_to_num(L2)
         assert torch.max(torch.abs(L1 - L2)).item() <= tol * torch.max(torch.abs(L1)).item(), kind
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("m,n", [(16384, 65), (16385, 65), (32768, 33), (32769, 17), (65536, 17), (65537, 9),
+                                 (131072, 9)])
+def test_tall_panels(nla, split_rows, dtype, m, n):
+    """Heights where the panel's columns change (64, 32, 16 and 8), one column
+    more than the narrowest of them takes: the pivots and factors of the
+    global-memory leaf."""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + n)
+    A0 = torch.empty((n, m), dtype=dtype, device=DEV).normal_(generator=g).t()
+    split_rows(0)
+    L1, p1, i1 = nla.getrf2_(A0.clone())
+    split_rows(1)
+    L2, p2, i2 = nla.getrf2_(A0.clone())
+    assert i1 == i2 == 0
+    assert torch.equal(p1, p2)
+    tol = 1e-12 if dtype == torch.float64 else 1e-5
+    assert torch.max(torch.abs(L1 - L2)).item() <= tol * torch.max(torch.abs(L1)).item()
+
+
+def test_four_tall_factorizations_at_once(nla):
+    """Four streams, one LU each of heights from 9000 to 120000 rows: every
+    panel's groups find a place beside the others', so none waits for a group
+    that never starts (such a wait ends after about a second, far above the
+    whole call), and the results are those of one at a time."""
+    import time
+    g = torch.Generator(device=DEV)
+    g.manual_seed(4)
+    from nextla_amd import _lib
+    lib = _lib.load()
+    shapes = [(20000, 128), (32000, 128), (60000, 64), (120000, 32)]
+    A0 = [torch.empty((n, m), dtype=torch.float64, device=DEV).normal_(generator=g).t() for m, n in shapes]
+    ref = [nla.getrf2_(a.clone()) for a in A0]
+    streams = [torch.cuda.Stream() for _ in shapes]
+    took = []
+    for _ in range(4):
+        work = [a.clone() for a in A0]
+        piv = [torch.zeros(n, dtype=torch.int64, device=DEV) for _, n in shapes]
+        info = torch.zeros(4, dtype=torch.int64, device=DEV)
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        for i, (m, n) in enumerate(shapes):
+            assert lib.nla_getrf2(_lib.NLA_F64, m, n, work[i].data_ptr(), m, piv[i].data_ptr(), info[i:].data_ptr(),
+                                  streams[i].cuda_stream) == 0
+        torch.cuda.synchronize()
+        took.append(time.perf_counter() - t0)
+        for i, (L, p, inf) in enumerate(ref):
+            assert info[i].item() == inf == 0 and torch.equal(piv[i], p) and torch.equal(work[i], L)
+    assert min(took) < 0.5, took
