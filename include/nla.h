@@ -218,8 +218,8 @@ int32_t nla_trmm(char side, char uplo, char transa, char diag, int32_t dtype, do
 /*
  * Recursive LU factorization with partial pivoting, A = P·L·U, in place
  * (replaces getrf2!(A, ipiv, info), src/lu.jl:185-300: LAPACK dgetrf2's
- * recursion).  Splits the columns at n1 = min(m,n)/2, factors the left
- * block, applies its interchanges to the right block, solves
+ * recursion).  Splits the columns at n1 = min(m,n)/2 (rounded up to whole
+ * panels), factors the left block, applies its interchanges to the right block, solves
  * A12 = L11^-1·A12 with the unit-lower TRSM of this library (nla_trsm,
  * diag 'U'), updates A22 -= A21·A12 (nla_gemm), factors A22 and applies its
  * interchanges to the left block; a panel of up to 64 columns is one kernel
@@ -228,12 +228,19 @@ int32_t nla_trmm(char side, char uplo, char transa, char diag, int32_t dtype, do
  *   ipiv  device array of min(m,n) int64: row i was interchanged with row
  *         ipiv[i] (1-based, as the reference);
  *   info  device int64: 0, or the 1-based index of the first exactly zero
- *         pivot (the factorization still completes, as LAPACK's); -1 if a
- *         leaf spread over several work-groups (NLA_CFG_LU_SPLIT_ROWS) timed
- *         out waiting for the others, when the factors are not valid.
+ *         pivot (the factorization still completes, as LAPACK's).
  * Enqueued on `stream`, no host synchronization.  Differences from the
  * reference: info is returned (the reference's Int argument cannot carry
  * it out), and the factorization does not stop at a zero pivot.
+ * Panels of more than one work-group (above 128 rows) exchange rows through a
+ * buffer of the (device, stream), allocated on first use and kept until the
+ * process ends: 2.4 MB for blocks of up to 4096 rows, 8.7 MB for taller ones;
+ * the triangular solves use the stream's workspace as nla_trsm does.  Host
+ * threads may share a stream.  Under graph capture a call of up to 4096 rows
+ * and 65 columns uses neither: it needs no call before it, and its graph may
+ * run beside others.  Other captured calls want a call of their size on that
+ * stream before (which allocates), and their graph must not run at the same
+ * time as another LU or solve of the stream that it was captured on.
  * Argument positions: 1 dtype, 2 m, 3 n, 4 A, 5 lda, 6 ipiv, 7 info,
  * 8 stream.
  */

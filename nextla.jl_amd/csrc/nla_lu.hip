@@ -358,7 +358,7 @@ constexpr int SYNC_WORDS = SYNC_SLOTS + 2 * PAR_WORDS;
 template <typename T>
 constexpr int64_t PANEL_M_MAX = sizeof(T) == 8 ? 64 * 256 : 128 * 256;
 constexpr int64_t PANEL_M_ALL = 131072;  // rows of any panel
-constexpr int64_t SYNC_BYTES = SYNC_WORDS * 8 + PANEL_M_MAX<double> * 64 * 8;
+constexpr int64_t SAVE_BYTES = PANEL_M_MAX<double> * 64 * 8;
 static_assert(PANEL_M_MAX<double> * 8 == PANEL_M_MAX<float> * 4, "one buffer serves both types");
 constexpr int64_t SPLIT_SPIN_LIMIT = int64_t(1) << 20;  // about a second of polling
 
@@ -962,15 +962,17 @@ __global__ void info_zero_kernel(int64_t *info) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *info = 0;
 }
 
-// Exchange slots and saved block of the register panels, one buffer per
-// (device, stream): launches on one stream run in order, so they share it.  A
-// panel and the recovery launch that follows it are enqueued under the
-// buffer's lock: with another host thread's panel in between, the recovery
-// would find that panel's block saved.
+// Exchange slots and saved block of the register panels, two buffers per
+// (device, stream), one for panels of up to SMALL_ROWS rows (2.4 MB) and one for
+// taller ones (8.7 MB), each allocated when first needed and kept: launches on
+// one stream run in order, so they share it.  A panel and the recovery launch
+// that follows it are enqueued under the lock: with another host thread's panel
+// in between, the recovery would find that panel's block saved.
+constexpr int64_t SMALL_ROWS = 4096;
 struct PanelSync {
     int dev;
     hipStream_t stream;
-    uint64_t *ptr = nullptr;
+    uint64_t *ptr[2] = {nullptr, nullptr};
     std::mutex mu;
 };
 
@@ -986,21 +988,38 @@ PanelSync *panel_sync(hipStream_t s, int32_t *st) {
     std::lock_guard<std::mutex> g(mu);
     for (auto &c : cache)
         if (c->dev == dev && c->stream == s) return c.get();
-    uint64_t *p = nullptr;
-    e = hipMalloc((void **)&p, SYNC_BYTES);
+    cache.emplace_back(new PanelSync());
+    cache.back()->dev = dev;
+    cache.back()->stream = s;
+    return cache.back().get();
+}
+
+// The buffer for m rows, called with sync->mu held.
+uint64_t *panel_buffer(PanelSync *sync, int64_t m, int32_t *st) {
+    uint64_t *&p = sync->ptr[m <= SMALL_ROWS ? 0 : 1];
+    if (p != nullptr) return p;
+    uint64_t *q = nullptr;
+    const int64_t save = m <= SMALL_ROWS ? SMALL_ROWS * 64 * 8 : SAVE_BYTES;
+    hipError_t e = hipMalloc((void **)&q, SYNC_WORDS * 8 + save);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(sync_zero_kernel, dim3(1), dim3(256), 0, s, p, SYNC_WORDS);
+        hipLaunchKernelGGL(sync_zero_kernel, dim3(1), dim3(256), 0, sync->stream, q, SYNC_WORDS);
         e = hipGetLastError();
     }
     if (e != hipSuccess) {
         *st = report_hip(e, "lu panel sync buffer");
         return nullptr;
     }
-    cache.emplace_back(new PanelSync());
-    cache.back()->dev = dev;
-    cache.back()->stream = s;
-    cache.back()->ptr = p;
-    return cache.back().get();
+    return p = q;
+}
+
+bool is_captured(hipStream_t s) {
+    if (s == nullptr) return false;  // the null stream cannot be
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st != hipStreamCaptureStatusNone;
 }
 
 template <typename T>
@@ -1011,6 +1030,7 @@ struct LuRec {
     hipStream_t s;
     int32_t st = NLA_OK;
     int64_t split_rows = lu_split_rows();
+    bool stateless = false;  // blocks of 129 to REG_ROWS rows in the register leaf: nothing shared, nothing allocated
     int64_t spin_limit = lu_spin_limit() > 0 ? lu_spin_limit() : SPLIT_SPIN_LIMIT;
 
     // the register panel for up to MOST rows
@@ -1028,11 +1048,13 @@ struct LuRec {
         PanelSync *sync = panel_sync(s, &st);
         if (!sync) return;
         std::lock_guard<std::mutex> pair(sync->mu);
+        uint64_t *buf = panel_buffer(sync, m, &st);
+        if (!buf) return;
         hipLaunchKernelGGL((lu_panel_kernel<T, NB, R, NT, false>), dim3(g), dim3(NT), 0, s, (int)m, n, A, lda, ipiv,
-                           info, r0, sync->ptr, spin_limit);
+                           info, r0, buf, spin_limit);
         if (!ok(hipGetLastError(), "lu panel")) return;
         hipLaunchKernelGGL(lu_panel_recover_kernel<T>, dim3(1), dim3(PIV_THREADS), 0, s, m, n, A, lda, ipiv, info, r0,
-                           sync->ptr);
+                           buf);
         ok(hipGetLastError(), "lu panel recovery");
     }
 
@@ -1091,14 +1113,31 @@ struct LuRec {
         }
     }
 
+    // The whole factorization.  A captured call must not allocate, and its
+    // graph may run beside others of its stream: its blocks of up to REG_ROWS
+    // rows take no exchange buffer if the stream has none for them yet, or if
+    // the call is thin (up to 65 columns; past them it has a triangular solve,
+    // whose workspace is the stream's in any case).  The register leaf takes up
+    // to 3 times as long as the panels there (1000 x 64 FP64 420 / 166 us).
+    void run(int64_t m, int64_t n, T *A, int64_t *ipiv) {
+        if (is_captured(s)) {
+            PanelSync *sync = panel_sync(s, &st);
+            if (!sync) return;
+            std::lock_guard<std::mutex> g(sync->mu);
+            stateless = (m <= REG_ROWS && std::min(m, n) <= 65) || sync->ptr[0] == nullptr;
+        }
+        rec(m, n, A, ipiv, 0);
+    }
+
     // Factor the m x n block at A, whose first row and column are the global
     // row / column r0 (blocks start on the diagonal); its pivots go to
     // ipiv[0 .. min(m,n)) as global 1-based rows, which is what the
     // reference's "ipiv[i] += n1" (src/lu.jl:289-291) makes of them.
     void rec(int64_t m, int64_t n, T *A, int64_t *ipiv, int64_t r0) {
         if (st != NLA_OK || m == 0 || n == 0) return;
-        const int nb = split_rows > 0 && m >= split_rows ? panel_cols<T>(m) : 0;
-        if (nb > 0 && narrow(m, n)) {
+        const bool regs = split_rows > 0 && m >= split_rows, leaf = m > 128 && m <= REG_ROWS && stateless;
+        const int nb = regs && !leaf ? panel_cols<T>(m) : 0;
+        if (regs && (leaf ? n <= LEAF_COLS : narrow(m, n))) {
             hipLaunchKernelGGL(lu_leaf_reg_kernel<T>, dim3(1), dim3(REG_THREADS), 0, s, (int)m, (int)n, A, lda, ipiv,
                                info, r0);
             ok(hipGetLastError(), "lu register leaf");
@@ -1169,10 +1208,10 @@ extern "C" int32_t nla_getrf2(int32_t dtype, int64_t m, int64_t n, void *A, int6
     if (m == 0 || n == 0) return NLA_OK;
     if (dtype == NLA_F64) {
         LuRec<double> r{dtype, lda, info, s};
-        r.rec(m, n, (double *)A, ipiv, 0);
+        r.run(m, n, (double *)A, ipiv);
         return r.st;
     }
     LuRec<float> r{dtype, lda, info, s};
-    r.rec(m, n, (float *)A, ipiv, 0);
+    r.run(m, n, (float *)A, ipiv);
     return r.st;
 }

@@ -395,3 +395,43 @@ def test_four_tall_factorizations_at_once(nla):
         for i, (L, p, inf) in enumerate(ref):
             assert info[i].item() == inf == 0 and torch.equal(piv[i], p) and torch.equal(work[i], L)
     assert min(took) < 0.5, took
+
+
+@pytest.mark.parametrize("m,n", [(1000, 64), (4096, 33), (300, 8), (100, 64)])
+def test_thin_graphs_of_one_stream_at_once(nla, m, n):
+    """Captured without a call before on a new stream; two graphs of the stream
+    replayed at once, with eager factorizations on that stream in between: every
+    replay gives the same factors, and the eager pivots."""
+    from nextla_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m * n)
+    A0 = [torch.empty((n, m), dtype=torch.float64, device=DEV).normal_(generator=g).t() for _ in range(2)]
+    ref = [nla.getrf2_(a.clone()) for a in A0]
+    work = [a.clone() for a in A0]
+    piv = [torch.zeros(min(m, n), dtype=torch.int64, device=DEV) for _ in A0]
+    info = torch.zeros(2, dtype=torch.int64, device=DEV)
+    home, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graphs = []
+    for i in range(2):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=home):
+            work[i].copy_(A0[i])
+            assert lib.nla_getrf2(_lib.NLA_F64, m, n, work[i].data_ptr(), m, piv[i].data_ptr(), info[i:].data_ptr(),
+                                  torch.cuda.current_stream().cuda_stream) == 0
+        graphs.append(graph)
+    first = None
+    for rep in range(6):
+        for i, st in enumerate((home, other)):
+            with torch.cuda.stream(st):
+                graphs[i].replay()
+        torch.cuda.synchronize()
+        if first is None:
+            first = [w.clone() for w in work]
+        for i in range(2):
+            assert info[i].item() == 0 and torch.equal(piv[i], ref[i][1]) and torch.equal(work[i], first[i])
+            scale = torch.max(torch.abs(ref[i][0])).item()
+            assert torch.max(torch.abs(work[i] - ref[i][0])).item() <= 1e-12 * scale
+        with torch.cuda.stream(home):
+            nla.getrf2_(A0[0].clone())

@@ -38,3 +38,36 @@ def test_panel_and_its_recovery_stay_together(lu, threads):
     assert len(users) == 2 * 3 * threads
     for panel, recover in zip(users[::2], users[1::2]):
         assert is_panel(panel) and not is_panel(recover) and panel[0] == recover[0], users
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("m,n", [(129, 64), (1000, 64), (4096, 33), (4096, 1), (128, 64), (700, 65), (40, 4096)])
+def test_thin_factorization_is_captured_on_a_new_stream(lu, dtype, m, n):
+    """A captured call on a stream that has factored nothing: no allocation
+    (which a capture does not allow) and no launch that uses the stream's
+    exchange buffer, so that graphs of such calls may run side by side."""
+    before = lu.emu_allocated()
+    st, log = launches(lu, dtype, m, n, stream=1000 + m + n, capturing=1)
+    assert st == 0 and lu.emu_allocated() == before
+    assert not any(is_panel(row) or "recover" in row[2] for row in log)
+    assert log
+
+
+def test_captured_after_a_call_of_its_size(lu):
+    """With the stream's buffer there, a wide captured call uses the panels; a
+    thin one still shares nothing."""
+    assert launches(lu, 1, 1000, 700, stream=5000)[0] == 0
+    st, log = launches(lu, 1, 1000, 700, stream=5000, capturing=1)
+    assert st == 0 and any(is_panel(row) for row in log)
+    st, log = launches(lu, 1, 1000, 64, stream=5000, capturing=1)
+    assert st == 0 and not any(is_panel(row) for row in log)
+    # a tall thin call has left the buffer of tall blocks only
+    assert launches(lu, 1, 5000, 64, stream=5001)[0] == 0
+    assert launches(lu, 1, 5000, 2000, stream=5001, capturing=1)[0] == 0
+
+
+def test_buffer_of_small_factorizations(lu):
+    """Up to 4096 rows a stream's buffer stays below 3 MB."""
+    before = lu.emu_allocated()
+    assert launches(lu, 1, 4096, 100, stream=6000)[0] == 0
+    assert 0 < lu.emu_allocated() - before < 3 << 20
