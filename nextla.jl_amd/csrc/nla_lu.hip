@@ -20,6 +20,7 @@
 #include <limits>
 #include <memory>
 #include <mutex>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -972,6 +973,7 @@ constexpr int64_t SMALL_ROWS = 4096;
 struct PanelSync {
     int dev;
     hipStream_t stream;
+    std::thread::id thread;  // hipStreamPerThread is another stream in every thread
     uint64_t *ptr[2] = {nullptr, nullptr};
     std::mutex mu;
 };
@@ -985,12 +987,14 @@ PanelSync *panel_sync(hipStream_t s, int32_t *st) {
         *st = report_hip(e, "lu panel device");
         return nullptr;
     }
+    const std::thread::id me = s == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id();
     std::lock_guard<std::mutex> g(mu);
     for (auto &c : cache)
-        if (c->dev == dev && c->stream == s) return c.get();
+        if (c->dev == dev && c->stream == s && c->thread == me) return c.get();
     cache.emplace_back(new PanelSync());
     cache.back()->dev = dev;
     cache.back()->stream = s;
+    cache.back()->thread = me;
     return cache.back().get();
 }
 

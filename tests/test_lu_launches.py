@@ -71,3 +71,13 @@ def test_buffer_of_small_factorizations(lu):
     before = lu.emu_allocated()
     assert launches(lu, 1, 4096, 100, stream=6000)[0] == 0
     assert 0 < lu.emu_allocated() - before < 3 << 20
+
+
+def test_threads_have_buffers_of_their_own_for_their_own_streams(lu):
+    """hipStreamPerThread is one handle for a different stream in every thread:
+    their panels run at the same time and must not share a buffer."""
+    before = lu.emu_allocated()
+    assert launches(lu, 1, 600, 64, threads=1, stream=7000)[0] == 0
+    one = lu.emu_allocated() - before
+    assert launches(lu, 1, 600, 64, threads=3, stream=2)[0] == 0
+    assert lu.emu_allocated() - before == 4 * one
