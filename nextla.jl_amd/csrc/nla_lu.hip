@@ -821,13 +821,18 @@ __global__ void laswp_kernel(int64_t ncols, T *__restrict__ A, int64_t lda, int6
 // each final row comes from and then permutes its columns.
 //
 // What was at position q before swap k came there with the latest earlier
-// swap j that targets q (from position j before swap j), or was there from
-// the start.  So every position's source is a short walk of its own over
-// lists of the swaps that target a position, all positions at once: composing
-// the swaps in order, one LDS round trip each, took 0.1 us per swap (430 us
-// for the 4096 of a half of n = 8192, 6 of LU's 43 ms there).  Then every
-// thread moves up to LASWP_R entries at a time, several columns per pass where
-// few rows move: all loads, a barrier, the stores.
+// swap j that targets q (from position j before swap j, and so on from there),
+// or was there from the start.  The swaps that target j all come before swap j,
+// so past the first step the latest of them all is the one: head.  The first
+// step needs the latest one before k with the same target: the swaps go in in
+// batches of one per thread, linked by target, and each looks for its
+// predecessor in its batch, or takes what head held before the batch.  Every
+// position's source is then a short walk of its own, all positions at once:
+// composing the swaps in order, one LDS round trip each, took 0.1 us per swap
+// (430 us for the 4096 of a half of n = 8192), and without batches a matrix whose
+// pivots are all the same row (a cyclic shift) cost each swap a walk along all
+// of them.  Then every thread moves up to LASWP_R entries at a time, several
+// columns per pass where few rows move: all loads, a barrier, the stores.
 constexpr int LASWP_THREADS = 1024, LASWP_R = 16, LASWP_COLS = 4;
 constexpr int LASWP_LDS = 163840 - 64;  // bytes: 4 per row of the block, 10 per swap
 constexpr int LASWP_SPAN = 38912;       // rows (a source is 16 bits, and LDS holds 812 swaps beside them)
@@ -843,9 +848,9 @@ __global__ __launch_bounds__(LASWP_THREADS) void laswp_perm_kernel(int64_t ncols
                                                                    const int64_t *__restrict__ ipiv, int64_t r0) {
     __shared__ __attribute__((aligned(4))) char s_mem[LASWP_LDS];
     __shared__ int s_moved;
-    int *head = reinterpret_cast<int *>(s_mem);                      // position -> a swap that targets it, -1 none
+    int *head = reinterpret_cast<int *>(s_mem);                      // position -> the last swap that targets it, -1 none
     uint16_t *piv = reinterpret_cast<uint16_t *>(s_mem + 4 * span);  // swap -> its target
-    uint16_t *next = piv + K;                                        // swap -> another with the same target
+    uint16_t *next = piv + K;                                        // swap -> the latest before it with the same target
     uint16_t *src = next + K;                                        // position < K -> the row that ends there
     uint16_t *dst = src + K, *dsrc = dst + K;                        // rows past K that move, and their sources
     const int t = threadIdx.x;
@@ -853,33 +858,46 @@ __global__ __launch_bounds__(LASWP_THREADS) void laswp_perm_kernel(int64_t ncols
     for (int x = t; x < span; x += LASWP_THREADS) head[x] = -1;
     if (t == 0) s_moved = 0;
     __syncthreads();
-    for (int k = t; k < K; k += LASWP_THREADS) {
-        const int64_t q = ipiv[b + k] - 1 - r0 - b;
-        const int p = (q >= k && q < span) ? (int)q : k;  // pivots lie in [k, span)
-        piv[k] = (uint16_t)p;
-        const int old = atomicExch(&head[p], k);
-        next[k] = old < 0 ? NONE : (uint16_t)old;
-    }
-    __syncthreads();
-    // the row at position q before swap k
-    auto source = [&](int q, int k) {
-        for (;;) {
-            int j = -1;
-            for (int c = head[q]; c >= 0;) {
-                if (c < k && c > j) j = c;
+    for (int k0 = 0; k0 < K; k0 += LASWP_THREADS) {
+        const int k = k0 + t;
+        int p = k;
+        if (k < K) {
+            const int64_t q = ipiv[b + k] - 1 - r0 - b;
+            if (q >= k && q < span) p = (int)q;  // pivots lie in [k, span)
+            piv[k] = (uint16_t)p;
+            if (p != k) {  // a swap with itself moves nothing
+                const int old = atomicExch(&head[p], k);
+                next[k] = old < 0 ? NONE : (uint16_t)old;
+            }
+        }
+        __syncthreads();
+        int before = -1;
+        bool last = p != k;
+        if (last) {
+            for (int c = head[p]; c >= 0;) {
+                if (c < k && c > before) before = c;
+                if (c > k) last = false;
+                if (c < k0) break;  // what the position held before this batch
                 const uint16_t n = next[c];
                 c = n == NONE ? -1 : (int)n;
             }
-            if (j < 0) return q;
-            q = j;
-            k = j;
         }
+        __syncthreads();  // every link of the batch has been read
+        if (k < K) next[k] = before < 0 ? NONE : (uint16_t)before;
+        if (last) head[p] = k;
+        __syncthreads();
+    }
+    // the row at position q after the swaps so far that target it
+    auto source = [&](int q) {
+        for (int j = head[q]; j >= 0; j = head[q]) q = j;
+        return q;
     };
     for (int x = t; x < span; x += LASWP_THREADS) {
         if (x < K) {
-            src[x] = (uint16_t)source(piv[x], x);
+            const uint16_t j = next[x];
+            src[x] = (uint16_t)(piv[x] == x ? source(x) : (j == NONE ? (int)piv[x] : source((int)j)));
         } else if (head[x] >= 0) {
-            const int from = source(x, K);
+            const int from = source(x);
             if (from != x) {
                 const int at = atomicAdd(&s_moved, 1);
                 dst[at] = (uint16_t)x;

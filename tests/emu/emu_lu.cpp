@@ -93,5 +93,15 @@ int emu_getrf2(int dtype, int64_t m, int64_t n, int threads, int64_t stream, int
         if (s != 0) return s;
     return 0;
 }
+// Interchanges b + 1 .. b + K (1-based rows in ipiv) of one block of rows on
+// the device kernel, its waves in either order.
+int emu_laswp(int64_t ncols, double *A, int64_t lda, int64_t b, int K, int span, const int64_t *ipiv, int reversed) {
+    std::vector<int> order;
+    for (int w = 0; w < nla::LASWP_THREADS / 64; ++w) order.push_back(reversed ? nla::LASWP_THREADS / 64 - 1 - w : w);
+    return emu::run(nla::LASWP_THREADS, 0, 1, order,
+                    [&] { nla::laswp_perm_kernel<double>(ncols, A, lda, b, K, span, ipiv, 0); })
+               ? 0
+               : 1;
+}
 int64_t emu_allocated(void) { return g_log.bytes; }
 }

@@ -3,9 +3,10 @@ tests/emu/emu_lu.cpp): how several host threads share a stream's exchange
 buffer, and which calls need one."""
 import ctypes
 
+import numpy as np
 import pytest
 
-from test_kernel_order import build
+from test_kernel_order import build, ptr
 
 
 @pytest.fixture(scope="module")
@@ -81,3 +82,30 @@ def test_threads_have_buffers_of_their_own_for_their_own_streams(lu):
     one = lu.emu_allocated() - before
     assert launches(lu, 1, 600, 64, threads=3, stream=2)[0] == 0
     assert lu.emu_allocated() - before == 4 * one
+
+
+def pivots(kind, m, b, K, rng):
+    k = np.arange(b, b + K)
+    p = {"random": lambda: rng.integers(k, m), "same": lambda: np.full(K, m - 1), "next": lambda: np.minimum(k + 1, m - 1),
+         "self": lambda: k, "few": lambda: np.maximum(k, rng.choice([m - 1, m // 2, m - 7], K)),
+         "near": lambda: np.minimum(k + rng.integers(0, 4, K), m - 1),
+         "back": lambda: np.maximum(k, m - 1 - k)}[kind]()
+    return p + 1
+
+
+@pytest.mark.parametrize("m,b,K", [(5, 0, 5), (700, 0, 64), (1500, 100, 1024), (1500, 3, 1025), (3000, 0, 2500)])
+@pytest.mark.parametrize("kind", ["random", "same", "next", "self", "few", "near", "back"])
+def test_interchanges_composed(lu, kind, m, b, K):
+    """The kernel that applies K interchanges as one permutation against the
+    swaps one after the other, for scattered, repeated and chained targets."""
+    rng = np.random.default_rng(m + K)
+    ipiv = np.zeros(m, np.int64)
+    ipiv[b:b + K] = pivots(kind, m, b, K, rng)
+    ref = np.arange(3 * m, dtype=np.float64).reshape(3, m)
+    got = [ref.copy() for _ in range(2)]
+    for i in range(b, b + K):
+        j = ipiv[i] - 1
+        ref[:, [i, j]] = ref[:, [j, i]]
+    for rev, g in enumerate(got):
+        assert lu.emu_laswp(ctypes.c_int64(3), ptr(g), ctypes.c_int64(m), ctypes.c_int64(b), K, m - b, ptr(ipiv), rev) == 0
+        assert np.array_equal(g, ref), kind
