@@ -579,9 +579,9 @@ int32_t nla_serve_destroy(nla_server server);
  *                      4096 columns eight-wave panels take 32 where that is
  *                      faster) or 32;
  *   NLA_CFG_PANEL_WAVES: waves per panel work-group (panels up to 512 rows):
- *                      4 (left-looking, 16 columns, two and more groups per
+ *                      4 (left-looking, two and more groups of 16 columns per
  *                      CU) or 8 (32-row units, right-looking TRSM); 0
- *                      (default) by the panel's rows and columns;
+ *                      (default) by the panel's rows, layout and columns;
  *   NLA_CFG_BATCH_CLASSES: size classes new batch plans may use, bit c for
  *                      systems up to 128 << c rows (c = 0..3; the 1024 class
  *                      is always on; default 0x1F: all, with bit 4).  A system goes to the

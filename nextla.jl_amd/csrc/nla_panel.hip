@@ -1099,20 +1099,26 @@ static hipError_t launch_panel_w(const PanelArgs<T> &a, hipStream_t s) {
     return kc ? launch_panel_k<T, 512, W, true>(a, s) : launch_panel_k<T, 512, W, false>(a, s);
 }
 
-template <typename T, int NBIG, bool TRMM>
+template <typename T, int NBIG, int WS, bool TRMM>
 static hipError_t launch_panel_left(const PanelArgs<T> &a, hipStream_t s) {
-    hipLaunchKernelGGL((panel_left_kernel<T, NBIG, 16, TRMM>), dim3((unsigned)((a.m + 15) / 16)), dim3(256), 0, s,
+    hipLaunchKernelGGL((panel_left_kernel<T, NBIG, WS, TRMM>), dim3((unsigned)((a.m + WS - 1) / WS)), dim3(256), 0, s,
                        a.nbig, a.m, a.M, a.mrs, a.mcs, a.lower ? 1 : 0, a.unit ? 1 : 0, a.B, a.brs, a.bcs, a.W, a.wrs,
                        a.wcs, a.scale, TRMM ? nullptr : a.F, TRMM ? nullptr : a.xmax);
     return hipGetLastError();
 }
 
+// 32 columns only where the setting asks for them; above 512 rows FP64's do not
+// fit LDS.
 template <typename T, bool TRMM>
 static hipError_t launch_panel_left_n(const PanelArgs<T> &a, hipStream_t s) {
-    if (a.nbig <= 128) return launch_panel_left<T, 128, TRMM>(a, s);
-    if (a.nbig <= 256) return launch_panel_left<T, 256, TRMM>(a, s);
-    if (a.nbig <= 512) return launch_panel_left<T, 512, TRMM>(a, s);
-    return launch_panel_left<T, 1024, TRMM>(a, s);
+    if (a.strip == 32) {
+        if (a.nbig <= 512) return launch_panel_left<T, 512, 32, TRMM>(a, s);
+        if constexpr (sizeof(T) == 4) return launch_panel_left<T, 1024, 32, TRMM>(a, s);
+    }
+    if (a.nbig <= 128) return launch_panel_left<T, 128, 16, TRMM>(a, s);
+    if (a.nbig <= 256) return launch_panel_left<T, 256, 16, TRMM>(a, s);
+    if (a.nbig <= 512) return launch_panel_left<T, 512, 16, TRMM>(a, s);
+    return launch_panel_left<T, 1024, 16, TRMM>(a, s);
 }
 
 // Right-hand sides per group of the eight-wave panel, or 0 for the
