@@ -10,8 +10,7 @@ device at hand and kept per device:
                       sides per work-group (16 or 32), per dtype
                       (NLA_CFG_PANEL_ROWS_*, NLA_CFG_PANEL_STRIP_*); a
                       tuned size replaces the library's default (0: 512
-                      rows where the panel's rows are contiguous in
-                      memory, 256 where they are strided) for every
+                      rows, or 256 by the panel's shape) for every
                       layout, so it is tuned on the layout that matters;
   batch classes       which LDS-sized variants of the persistent batched
                       solver a plan may use, and whether systems above 512
@@ -21,8 +20,8 @@ device at hand and kept per device:
 Each candidate is timed with HIP events on a representative problem (the
 8192 x 8192 drop-in case for panels; a 10,000-system-style mixed batch for
 the classes) and the fastest is applied with nla_set_config.  Results are
-cached as JSON per device name (NEXTLA_AMD_TUNE_CACHE, else
-~/.cache/nextla_amd/tune.json); tune() reuses a cached entry unless told
+cached as JSON per device name and generation of the kernels
+(NEXTLA_AMD_TUNE_CACHE, else ~/.cache/nextla_amd/tune.json); tune() reuses a cached entry unless told
 to measure again.  Every candidate gives results identical to the
 oracle's within the same bounds (tests/test_gpu_parity.py::test_panel_shapes,
 tests/test_gpu_batch.py::test_size_classes_bitwise_identical), so the tuner
@@ -37,6 +36,7 @@ from . import _lib
 PANEL_ROWS = (256, 384, 512)
 PANEL_STRIPS = (16, 32)
 BATCH_MASKS = (0x8, 0xC, 0xE, 0xF, 0x1E, 0x1F)  # 0x10: stage systems above 512 rows
+KERNELS = 2  # generation of the panel and batch kernels: a cached choice holds for the one it was measured on
 _KEYS = {"f32": (_lib.NLA_CFG_PANEL_ROWS_F32, _lib.NLA_CFG_PANEL_STRIP_F32),
          "f64": (_lib.NLA_CFG_PANEL_ROWS_F64, _lib.NLA_CFG_PANEL_STRIP_F64)}
 
@@ -108,7 +108,8 @@ def tune(device=None, force=False, dtypes=("f32", "f64"), save=True, apply_resul
     import torch
     dev = torch.device(device or "cuda")
     props = torch.cuda.get_device_properties(dev)
-    key = f"{props.name}|{getattr(props, 'gcnArchName', '')}|{props.multi_processor_count}"
+    key = (f"{props.name}|{getattr(props, 'gcnArchName', '')}|{props.multi_processor_count}"
+           f"|kernels {KERNELS}")
     path = cache_path()
     cache = {}
     if os.path.exists(path):
