@@ -15,6 +15,8 @@
 // unaligned 16-byte loads), so odd leading dimensions cost nothing here.
 #pragma once
 
+#include <limits>
+
 #include "nla_device.h"
 
 namespace nla {
@@ -231,13 +233,35 @@ __device__ __forceinline__ void split_tile(int64_t M, int64_t N, int64_t K, T al
 #pragma unroll
             for (int e = 0; e < 4; ++e) red[(w * NR + (c * RB + r) * 4 + e) * 64 + lane] = acc[c][r][e];
     __syncthreads();
+    bool odd = false;
 #pragma unroll
     for (int i = 0; i < NR / KS; ++i) {
         const int q = i * KS + w;
         T sum = red[q * 64 + lane];
 #pragma unroll
         for (int v = 1; v < KS; ++v) sum += red[(v * NR + q) * 64 + lane];
+        if (TRI) odd |= !(fabs(sum) <= std::numeric_limits<T>::max());
         if (in[i]) *d[i] = alpha * sum + cv[i];
+    }
+    if constexpr (TRI) {
+        // a zero that stands for one operand's other triangle, times an
+        // infinity or NaN of the other: such sums again, over their own k
+        // (beta is 0 here)
+        if (odd) {
+#pragma unroll 1
+            for (int q = w; q < NR; q += KS) {
+                const int64_t r = OX::outer(q / 4 % RB, lane & 15), c = OY::outer(q / (4 * RB), MM::di(lane, q % 4));
+                if (row0 + r >= M || col0 + c >= N) continue;
+                T *p = C + r + c * ldc;
+                if (fabs(*p) <= std::numeric_limits<T>::max()) continue;
+                const T *x = X + (TX ? (row0 + r) * ldx : row0 + r), *y = Y + (TY ? col0 + c : (col0 + c) * ldy);
+                T sum = T(0);
+#pragma unroll 1
+                for (int64_t k = row0 + r > col0 + c ? row0 + r : col0 + c; k < K; ++k)
+                    sum += x[TX ? k : k * ldx] * y[TY ? k * ldy : k];
+                *p = alpha * sum;
+            }
+        }
     }
 }
 
