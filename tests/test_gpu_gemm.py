@@ -67,3 +67,12 @@ def test_between_the_kernels(nla, dtype, m, n, k):
     """Shapes near the line between the K-splitting and the tiled kernels,
     long and narrow ones among them."""
     check(nla, dtype, m, n, k, (0, 3))
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(4095, 4095, 1501), (4093, 4090, 1504)])
+def test_largest_tiles_ragged(nla, dtype, m, n, k):
+    """Sizes that take the largest tiles (FP64 256 x 128, FP32 256 x 256 with a
+    loop of its own), ragged in M and N, with whole and partial k steps, odd
+    leading dimensions."""
+    check(nla, dtype, m, n, k, (0, 3))

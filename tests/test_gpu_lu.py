@@ -435,3 +435,26 @@ def test_thin_graphs_of_one_stream_at_once(nla, m, n):
             assert torch.max(torch.abs(work[i] - ref[i][0])).item() <= 1e-12 * scale
         with torch.cuda.stream(home):
             nla.getrf2_(A0[0].clone())
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("m,n", [(128, 64), (100, 33), (65, 64), (33, 40), (2, 2)])
+@pytest.mark.parametrize("value", [0.0, float("nan")])
+def test_single_group_panel_without_a_pivot(nla, split_rows, dtype, m, n, value):
+    """Up to 128 rows and 64 columns, one work-group: a column of zeros or of
+    NaN, the first and a later one: the info, pivots, factors and NaNs of the
+    global-memory leaf."""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + n)
+    for col in (0, min(m, n) - 1):
+        A0 = torch.empty((n, m), dtype=dtype, device=DEV).normal_(generator=g).t()
+        A0[:, col] = value
+        split_rows(0)
+        L1, p1, i1 = nla.getrf2_(A0.clone())
+        split_rows(1)
+        L2, p2, i2 = nla.getrf2_(A0.clone())
+        assert i1 == i2 == (col + 1 if value == 0.0 else 0) and torch.equal(p1, p2)
+        assert torch.equal(torch.isnan(L1), torch.isnan(L2))
+        tol = 1e-12 if dtype == torch.float64 else 1e-4
+        L1, L2 = torch.nan_to_num(L1), torch.nan_to_num(L2)
+        assert torch.max(torch.abs(L1 - L2)).item() <= tol * max(1.0, torch.max(torch.abs(L1)).item())
