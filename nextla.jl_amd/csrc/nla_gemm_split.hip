@@ -57,26 +57,28 @@ hipError_t launch_split(const GemmArgs<T> &a, hipStream_t s) {
 template <typename T>
 hipError_t launch_gemm(const GemmArgs<T> &a, hipStream_t s) {
     if (a.M <= 0 || a.N <= 0) return hipSuccess;
-    // Split where its estimated time is the shorter: q tiles of 32 x 32 per CU,
-    // each with a start and end of 0.6 us and the rate of its orientation (with
-    // op(X) transposed a lane loads from 16 rows of memory), against the rounds
-    // of the tiled kernels and the 1.6 us that their first and last steps take
-    // more.  Within 0.5 % of the faster one on average over K = 16 .. 4096 and
-    // 16 to 4096 tiles of 32 x 32, at most 10 % slower where the tiles are
-    // square and fill the last round.  Measured on MI355X (us per launch, tiled /
-    // split): FP64 64 x 4096 x 4096 371 / 50, 1024^3 89 / 48, 1536 x 1536 x 192
-    // 32.5 / 33.5, 1408 x 1408 x 192 22.9 / 30.2, 1024 x 1024 x 48 9.5 / 10.0,
-    // with X transposed 9.3 / 12.2, 1152 x 1152 x 192 so 21.4 / 30.5; FP32
-    // 512 x 512 x 192 6.6 / 4.8, 768 x 768 x 64 4.8 / 5.5, 768 x 768 x 1024
-    // 24 / 23, 256 x 4096 x 4096 97 / 118.
+    // Split where the tiles leave the chip idle and its estimated time is the
+    // shorter: q tiles of 32 x 32 per CU, each with a start and end of 0.6 us and
+    // the rate of its orientation (with op(X) transposed a lane loads from 16
+    // rows of memory), against the rounds of the tiled kernels and the 1.6 us
+    // that their first and last steps take more.  Measured on MI355X (us per
+    // launch, tiled / split): FP64 64 x 4096 x 4096 371 / 50, 1024^3 90 / 49,
+    // 1280 x 1280 x 512 49 / 42, 1408 x 1408 x 192 22.9 / 30.2, 1024 x 1024 x 48
+    // 9.3 / 10.0, with X transposed 9.3 / 12.2, 1152 x 1152 x 192 so 21.4 / 30.5,
+    // 1024 x 1024 x 1024 so 88 / 64; FP32 512 x 512 x 192 6.6 / 4.8, 768 x 768 x 64
+    // 4.8 / 5.5, 704 x 704 x 1024 24 / 16.  At most 10 % from the faster one
+    // over K = 16 .. 4096 and 16 to 4096 tiles of 32 x 32, 0.5 % on average.
     if (a.leaf == 0 && a.tri == 0 && a.K > 0) {
         constexpr bool F64 = sizeof(T) == 8;
-        const int64_t tiles = ((a.M + 31) / 32) * ((a.N + 31) / 32), q = (tiles + 255) / 256;
+        auto tiles = [&](int b) { return ((a.M + b - 1) / b) * ((a.N + b - 1) / b); };
+        const bool idle = F64 ? tiles(128) <= (a.K < 128 ? 64 : (a.tx ? 96 : 192)) : tiles(64) <= 144;
+        const int64_t q = (tiles(32) + 255) / 256;
         const double rate = F64 ? (a.tx ? (a.ty ? 0.0104 : 0.0150) : (a.ty ? 0.0090 : 0.0094))
                                 : (a.tx ? (a.ty ? 0.0070 : 0.0074) : 0.0062);  // us per k and tile of a CU
         double tiled = 0;
         gemm_tile_shape<T>(a.M, a.N, (a.K + 15) / 16 * 16, &tiled);
-        if ((double)q * (0.6 + rate * (double)(a.K + (F64 ? 16 : 32))) < tiled + 1.6) return launch_split<T, 2, 2, 4>(a, s);
+        if (idle && (double)q * (0.6 + rate * (double)(a.K + (F64 ? 16 : 32))) < tiled + 1.6)
+            return launch_split<T, 2, 2, 4>(a, s);
     }
     return launch_gemm_tiled<T>(a, s);
 }
