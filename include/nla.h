@@ -219,11 +219,11 @@ int32_t nla_trmm(char side, char uplo, char transa, char diag, int32_t dtype, do
  * Recursive LU factorization with partial pivoting, A = P·L·U, in place
  * (replaces getrf2!(A, ipiv, info), src/lu.jl:185-300: LAPACK dgetrf2's
  * recursion).  Splits the columns at n1 = min(m,n)/2 (rounded up to whole
- * panels), factors the left block, applies its interchanges to the right block, solves
- * A12 = L11^-1·A12 with the unit-lower TRSM of this library (nla_trsm,
- * diag 'U'), updates A22 -= A21·A12 (nla_gemm), factors A22 and applies its
- * interchanges to the left block; a panel of up to 64 columns is one kernel
- * (pivot = first index of the largest |a|, swap, scale by the reciprocal).
+ * panels), factors the left block, applies its interchanges to the right
+ * block, solves A12 = L11^-1·A12 with the unit-lower TRSM of this library
+ * (nla_trsm, diag 'U'), updates A22 -= A21·A12 (nla_gemm), factors A22 and
+ * applies its interchanges to the left block; a panel of up to 64 columns is
+ * one kernel (pivot = first index of the largest |a|, swap, scale by the reciprocal).
  *   A     m x n column-major (leading dimension lda), FP32 or FP64;
  *   ipiv  device array of min(m,n) int64: row i was interchanged with row
  *         ipiv[i] (1-based, as the reference);
@@ -251,7 +251,7 @@ int32_t nla_getrf2(int32_t dtype, int64_t m, int64_t n, void *A, int64_t lda, in
  * LAUUM: A := U·U^T (uplo 'U') or L^T·L (uplo 'L') in place, using and
  * writing only the uplo triangle (replaces lauum!(uplo, n, A, ib),
  * src/lauum.jl:52-186; the block size ib is internal here): one triangular
- * product in tiles, through the workspace in two or three runs (128 rows and
+ * product in tiles, through the workspace in two to four runs (128 rows and
  * less in one work-group).  What the other triangle holds plays no part.
  * The workspace (nla_lauum_workspace_bytes: (n/2 rounded up to 64)^2
  * elements) is the caller's; none is needed for n <= 128.
@@ -591,11 +591,13 @@ int32_t nla_serve_destroy(nla_server server);
  *                      512-row stages (panels of the 512 class plus a grouped
  *                      GEMM) instead of as one 1024-row panel.
  *   NLA_CFG_LU_SPLIT_ROWS: nla_getrf2 panels of at least this many rows are
- *                      held in registers: one work-group up to 128 rows,
- *                      above that up to 128 of them, to 131072 rows (default
- *                      1: every panel up to that size; 0 = 8-column blocks
- *                      in the one-work-group leaf that works in global
- *                      memory, for every size).
+ *                      held in registers: one work-group up to 128 rows, and
+ *                      up to 4096 with 8 columns and less; above that
+ *                      several, at most a quarter of the chip, to 131072
+ *                      rows (64 columns and fewer of them the taller it is)
+ *                      (default 1: every panel up to that size; 0 =
+ *                      8-column blocks in the one-work-group leaf that works
+ *                      in global memory, for every size).
  *   NLA_CFG_RESIDUAL:  residual of nla_rectrxm_mixed: NLA_RES_INT8 (default)
  *                      for n in [2048, 65536] and m >= 64, FP64 otherwise;
  *                      NLA_RES_FP64 for every size.  Read when the

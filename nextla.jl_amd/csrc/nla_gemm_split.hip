@@ -57,17 +57,19 @@ hipError_t launch_split(const GemmArgs<T> &a, hipStream_t s) {
 template <typename T>
 hipError_t launch_gemm(const GemmArgs<T> &a, hipStream_t s) {
     if (a.M <= 0 || a.N <= 0) return hipSuccess;
-    // Split where the tiles leave the chip idle and its estimated time is the
-    // shorter: q tiles of 32 x 32 per CU, each with a start and end of 0.6 us and
-    // the rate of its orientation (with op(X) transposed a lane loads from 16
-    // rows of memory), against the rounds of the tiled kernels and the 1.6 us
-    // that their first and last steps take more.  Measured on MI355X (us per
-    // launch, tiled / split): FP64 64 x 4096 x 4096 371 / 50, 1024^3 90 / 49,
-    // 1280 x 1280 x 512 49 / 42, 1408 x 1408 x 192 22.9 / 30.2, 1024 x 1024 x 48
-    // 9.3 / 10.0, with X transposed 9.3 / 12.2, 1152 x 1152 x 192 so 21.4 / 30.5,
-    // 1024 x 1024 x 1024 so 88 / 64; FP32 512 x 512 x 192 6.6 / 4.8, 768 x 768 x 64
-    // 4.8 / 5.5, 704 x 704 x 1024 24 / 16.  At most 10 % from the faster one
-    // over K = 16 .. 4096 and 16 to 4096 tiles of 32 x 32, 0.5 % on average.
+    // Split where few tiles leave the chip idle (`idle`; past it, as at 30000 x
+    // 32 x 1000 in FP64 where a split would take 49 us for 134, products keep the
+    // order of the tiles' sums) and its estimated time is the shorter: q tiles of
+    // 32 x 32 per CU, each with a start and end of 0.6 us and the rate of its
+    // orientation (with op(X) transposed a lane loads from 16 rows of memory),
+    // against the rounds of the tiled kernels and the 1.6 us that their first and
+    // last steps take more. Measured on MI355X (us per launch, tiled / split):
+    // FP64 64 x 4096 x 4096 371 / 50, 1024^3 90 / 49, 1280 x 1280 x 512 49 / 42,
+    // 1408 x 1408 x 192 22.9 / 30.2, 1024 x 1024 x 48 9.3 / 10.0, with X
+    // transposed 9.3 / 12.2, 1152 x 1152 x 192 so 21.4 / 30.5, 1024 x 1024 x 1024
+    // so 88 / 64; FP32 512 x 512 x 192 6.6 / 4.8, 768 x 768 x 64 4.8 / 5.5, 704 x
+    // 704 x 1024 24 / 16. At most 10 % from the faster one over K = 16 .. 4096
+    // and 16 to 4096 tiles of 32 x 32, 0.5 % on average.
     if (a.leaf == 0 && a.tri == 0 && a.K > 0) {
         constexpr bool F64 = sizeof(T) == 8;
         auto tiles = [&](int b) { return ((a.M + b - 1) / b) * ((a.N + b - 1) / b); };

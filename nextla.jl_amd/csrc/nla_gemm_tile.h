@@ -1,5 +1,5 @@
 // One tile of C = beta*C + alpha*op(X)*op(Y) on gfx950 MFMA, shared by the
-// GEMM update, the grouped GEMM of the batched solver and lauum's product.
+// GEMM update and the grouped GEMM of the batched solver.
 //
 // Orientation: the MFMA computes D = C^T for each 16x16 (f64) / 32x32 (f32)
 // block, so that the lane index of D's column walks down a column of C and the

@@ -8,7 +8,7 @@
 // A.  A tile of block row i reads the factor's rows from i down, in its own
 // block and in the diagonal block of that row; so in row order, diagonal tile
 // last, any run of tiles may be copied back before the next is computed, and
-// the workspace of about half the triangle's size takes two runs and a rest.
+// the workspace of about half the triangle's size takes two to four runs.
 // The recursion this replaces (a TRMM, a GEMM and a masked add per level, one
 // work-group per 128-row leaf) took 2.15 ms at n = 4096 in FP64.  Up to 128
 // rows are one work-group in LDS.

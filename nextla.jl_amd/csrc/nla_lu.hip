@@ -4,14 +4,14 @@
 // TRSM and GEMM update.
 //
 // The host walks the same recursion as the reference: split the columns at
-// n1 = min(m, n) / 2, factor the left block, apply its row interchanges to
+// n1 = min(m, n) / 2 (rounded up to whole panels), factor the left block, apply its row interchanges to
 // the right block, solve A12 = L11^-1 A12 (unit lower), update
 // A22 -= A21 A12, factor A22 and apply its interchanges to the left block.
 // Panels of up to 64 columns are one kernel (the same eliminations with
 // rank-1 updates in place of the GEMMs of that width), held in registers by
-// up to 128 work-groups that exchange one pivot row per column (fewer columns
-// from 16,384 rows on, in FP32 32,768; past 131,072 rows 8 columns in global
-// memory).  Pivots are kept as global rows throughout (the reference shifts
+// work-groups that exchange one pivot row per column and take at most a
+// quarter of the chip (fewer columns above 16,384 rows, in FP32 32,768; past
+// 131,072 rows 8 columns in global memory).  Pivots are kept as global rows throughout (the reference shifts
 // them by n1 after each recursive call).  Everything is enqueued on the
 // caller's stream; pivots and info stay on the device.
 #include <hip/hip_runtime.h>
